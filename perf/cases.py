@@ -171,7 +171,8 @@ class _Forces:
         mn, mx = np.array(c.maprealposmin), np.array(c.maprealposmax)
         nc = [int(v) for v in np.ceil((mx - mn) / float(ks))]
         bits = [max(2, (v + 1).bit_length()) for v in nc]
-        bits = [b + (31 - sum(bits)) // 3 for b in bits]
+        for i in range(31 - sum(bits)):   # all 31 bits are used, x first
+            bits[i % 3] += 1
         sx, sy, sz = bits
         t.cellcode = ((sx + 1) << 25 | sy << 20 | sz << 15 | (sy + sz) << 10 | (sx + 1 + sz) << 5 |
                       (sx + 1 + sy))
