@@ -11,7 +11,7 @@
 //   A (16x16, row-major MxK): lane holds A[c][4g..4g+3]
 //   B (16x16, KxN):           lane holds B[4g..4g+3][c]
 //   D (16x16, MxN):           lane holds D[4g..4g+3][c]
-// A tile is 16 samples (particles). A D-layout block of Z = X W^T (rows =
+// A tile is 16 samples (particles). Training: a D-layout block of Z = X W^T (rows =
 // samples, cols = units) is directly the A operand of the transposed block
 // (units x samples) and the B operand of (samples x units): the weight
 // gradients need no data movement; only dH1 = dZ2 W2 goes through LDS.
@@ -30,6 +30,7 @@ namespace {
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bfx4 __attribute__((ext_vector_type(4)));
 
 constexpr int kIn = 11, kInPad = 16, kHid = 64;
 // Offsets of the parameter block (FP32 master and gradients).
@@ -63,9 +64,8 @@ __device__ inline f32x4 mfma(bf16x4 a, bf16x4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
 }
 __device__ inline bf16x4 pack4(float a, float b, float c, float d) {
-  bf16x4 r;
-  r[0] = (short)f2bf(a); r[1] = (short)f2bf(b); r[2] = (short)f2bf(c); r[3] = (short)f2bf(d);
-  return r;
+  // Two v_cvt_pk_bf16_f32 (round to nearest even, as f2bf).
+  return __builtin_bit_cast(bf16x4, __builtin_convertvector(f32x4{a, b, c, d}, bfx4));
 }
 __device__ inline bf16x4 load_bf4(const unsigned short* p) {
   bf16x4 r;
@@ -166,31 +166,116 @@ __device__ inline void forward_tile(const unsigned short* __restrict__ wbf,
 }
 
 // ---------------------------------------------------------------- inference
+// The layers transposed: Z1^T = W1 X^T, Z2^T = W2 H1^T. A D-layout block of
+// Z1^T (rows = units, cols = samples) is, after SiLU, the B operand of the
+// next product as it stands, so nothing goes through LDS, and the last
+// layer's sum over units is within the lane but for the four lane groups.
+// The wave keeps weights and biases in registers for all its tiles.
+// Bound by the VALU's exp and reciprocal (32 SiLU a lane and tile): the quotient of
+// SiLU is a product with v_rcp_f32 (1 ulp). 1000003 samples: 103 us with weights
+// and H1 re-read for every tile and exact quotients, 39 us.
+struct FwdWeights {
+  bf16x4 w1[4], w2[4][4];
+  f32x4 b1[4], b2[4], w3[4];
+  float mean[4], scale[4], b3;
+};
+
+__device__ inline void load_weights(const unsigned short* __restrict__ wbf,
+                                    const float* __restrict__ par, const Norm& nm,
+                                    FwdWeights& w) {
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+#pragma unroll
+  for (int jb = 0; jb < 4; jb++) {
+    w.w1[jb] = load_bf4(wbf + kBfW1 + (jb * 16 + c) * kInPad + 4 * g);
+#pragma unroll
+    for (int kb = 0; kb < 4; kb++)
+      w.w2[jb][kb] = load_bf4(wbf + kBfW2 + (jb * 16 + c) * kHid + kb * 16 + 4 * g);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int u = jb * 16 + 4 * g + r;
+      w.b1[jb][r] = par[kOffB1 + u];
+      w.b2[jb][r] = par[kOffB2 + u];
+      w.w3[jb][r] = bf2f(wbf[kBfW3 + u]);
+    }
+  }
+  w.b3 = par[kOffB3];
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    w.mean[r] = nm.mean[4 * g + r];
+    w.scale[r] = nm.scale[4 * g + r];
+  }
+}
+
+__device__ inline float fast_silu(float z) { return z * fast_rcp(1.f + __expf(-z)); }
+
+// Network output (before softplus) of sample c of a tile of 16, on all lanes of
+// column c. feat(i, k): raw feature k of sample i.
+template <typename FeatFn>
+__device__ inline float forward_tile_t(const FwdWeights& w, FeatFn feat) {
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+  float x[4];
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int k = 4 * g + r;
+    x[r] = k < kIn ? (feat(c, k) - w.mean[r]) * w.scale[r] : 0.f;
+  }
+  const bf16x4 bx = pack4(x[0], x[1], x[2], x[3]);
+  bf16x4 h[4];
+#pragma unroll
+  for (int jb = 0; jb < 4; jb++) {
+    const f32x4 z = mfma(w.w1[jb], bx, w.b1[jb]);
+    h[jb] = pack4(fast_silu(z[0]), fast_silu(z[1]), fast_silu(z[2]), fast_silu(z[3]));
+  }
+  float o = 0.f;
+#pragma unroll
+  for (int jb = 0; jb < 4; jb++) {
+    f32x4 z = w.b2[jb];
+#pragma unroll
+    for (int kb = 0; kb < 4; kb++) z = mfma(w.w2[jb][kb], h[kb], z);
+#pragma unroll
+    for (int r = 0; r < 4; r++) o += fast_silu(z[r]) * w.w3[jb][r];
+  }
+  return across_groups_sum(o) + w.b3;
+}
+
+// Runs the network over samples [0, n), 16 kT samples per wave and turn, and
+// calls done(sample, o) once per sample. kT = 4: lane group g finishes tile g
+// (whole waves store); kT = 1 spreads small batches over more waves.
+template <int kT, typename FeatFn, typename DoneFn>
+__device__ inline void forward_all(unsigned n, const unsigned short* __restrict__ wbf,
+                                   const float* __restrict__ par, const Norm& nm, FeatFn feat,
+                                   DoneFn done) {
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+  FwdWeights w;
+  load_weights(wbf, par, nm, w);
+  const unsigned nturns = (n + 16 * kT - 1) / (16 * kT);
+  for (unsigned t = blockIdx.x; t < nturns; t += gridDim.x) {
+    const unsigned base = t * 16 * kT;
+    float o = 0.f;
+#pragma unroll 1
+    for (int k = 0; k < kT; k++) {
+      const float ok = forward_tile_t(w, [&](int i, int j) { return feat(base + 16 * k + i, j); });
+      o = g == k ? ok : o;
+    }
+    if (g < kT && base + 16 * g + c < n) done(base + 16 * g + c, o);
+  }
+}
+
+// Resident waves of the inference kernels (4 per SIMD of 256 CUs); up to so many
+// tiles each wave takes one tile.
+constexpr unsigned kFwdWaves = 4096;
+
 // nu[i] = out_scale * softplus(MLP(features[i])) for i in [0,n); features are
 // [n][11] FP32 rows.
-__global__ void __launch_bounds__(64) k_mlp_forward(unsigned n, const float* __restrict__ feat,
+template <int kT>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8)))
+k_mlp_forward(unsigned n, const float* __restrict__ feat,
     const unsigned short* __restrict__ wbf, const float* __restrict__ par, Norm nm,
     float* __restrict__ out) {
-  __shared__ unsigned short lds_h1[16 * kHid];
-  const unsigned ntiles = (n + 15) / 16;
-  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-  for (unsigned t = blockIdx.x; t < ntiles; t += gridDim.x) {
-    const unsigned base = t * 16;
-    auto fe = [&](int i, int k) -> float {
-      const unsigned s = base + i;
-      return s < n ? feat[size_t(s) * kIn + k] : 0.f;
-    };
-    Fwd f;
-    forward_tile(wbf, par, nm, fe, lds_h1, f);
-    if (c == 0) {
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const unsigned s = base + 4 * g + r;
-        if (s < n) out[s] = nm.out_scale * softplus(f.o[r]);
-      }
-    }
-    __syncthreads();
-  }
+  forward_all<kT>(
+      n, wbf, par, nm,
+      [&](unsigned s, int k) { return s < n ? feat[size_t(s) * kIn + k] : 0.f; },
+      [&](unsigned s, float o) { out[s] = nm.out_scale * softplus(o); });
 }
 
 // ---------------------------------------------------------------- training
@@ -413,51 +498,38 @@ __global__ void __launch_bounds__(256) k_mlp_to_bf16(const float* __restrict__ p
 // the velocity gradient G[9] of the interaction, rho and dp; nu_t replaces
 // smag*sqrt(prr) of KerComputeSpsTau (JSphGpu_ker.cu:1387-1436); the
 // isotropic blin term is kept.
-__global__ void __launch_bounds__(64) k_sps_tau_learned(unsigned n, unsigned pini, float blin,
+template <int kT>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8)))
+k_sps_tau_learned(unsigned n, unsigned pini, float blin,
     float dp, const float4* __restrict__ velrho, const float* __restrict__ velgrad,
     const float* __restrict__ s2, const unsigned short* __restrict__ wbf,
     const float* __restrict__ par, Norm nm, float* __restrict__ tau, float* __restrict__ nu_out) {
-  __shared__ unsigned short lds_h1[16 * kHid];
-  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-  const unsigned ntiles = (n + 15) / 16;
-  for (unsigned t = blockIdx.x; t < ntiles; t += gridDim.x) {
-    const unsigned base = t * 16;
-    auto fe = [&](int i, int k) -> float {
-      const unsigned s = base + i;
-      if (s >= n) return 0.f;
-      const unsigned p = s + pini;
-      if (k < 9) return velgrad[9 * size_t(p) + k];
-      return k == 9 ? velrho[p].w : dp;
-    };
-    Fwd f;
-    forward_tile(wbf, par, nm, fe, lds_h1, f);
-    if (c == 0) {
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const unsigned s = base + 4 * g + r;
-        if (s >= n) continue;
-        const unsigned p = s + pini;
-        const float visc_sps = nm.out_scale * softplus(f.o[r]);
-        const float* sp = s2 + 6 * size_t(p);
-        const float xx = sp[0], xy = sp[1], xz = sp[2], yy = sp[3], yz = sp[4], zz = sp[5];
-        const float pow1 = xx * xx + yy * yy + zz * zz;
-        const float prr = xy * xy + xz * xz + yz * yz + pow1 + pow1;
-        const float div_u = xx + yy + zz;
-        const float sumsps = -(visc_sps * div_u + blin * prr);
-        const float two = visc_sps + visc_sps;
-        const float one_rho = 1.0f / velrho[p].w;
-        float* tp = tau + 6 * size_t(p);
-        tp[0] = one_rho * (two * xx + sumsps);
-        tp[1] = one_rho * (visc_sps * xy);
-        tp[2] = one_rho * (visc_sps * xz);
-        tp[3] = one_rho * (two * yy + sumsps);
-        tp[4] = one_rho * (visc_sps * yz);
-        tp[5] = one_rho * (two * zz + sumsps);
-        if (nu_out) nu_out[p] = visc_sps;
-      }
-    }
-    __syncthreads();
-  }
+  auto feat = [&](unsigned s, int k) -> float {
+    if (s >= n) return 0.f;
+    const unsigned p = s + pini;
+    if (k < 9) return velgrad[9 * size_t(p) + k];
+    return k == 9 ? velrho[p].w : dp;
+  };
+  forward_all<kT>(n, wbf, par, nm, feat, [&](unsigned s, float o) {
+    const unsigned p = s + pini;
+    const float visc_sps = nm.out_scale * softplus(o);
+    const float* sp = s2 + 6 * size_t(p);
+    const float xx = sp[0], xy = sp[1], xz = sp[2], yy = sp[3], yz = sp[4], zz = sp[5];
+    const float pow1 = xx * xx + yy * yy + zz * zz;
+    const float prr = xy * xy + xz * xz + yz * yz + pow1 + pow1;
+    const float div_u = xx + yy + zz;
+    const float sumsps = -(visc_sps * div_u + blin * prr);
+    const float two = visc_sps + visc_sps;
+    const float one_rho = 1.0f / velrho[p].w;
+    float* tp = tau + 6 * size_t(p);
+    tp[0] = one_rho * (two * xx + sumsps);
+    tp[1] = one_rho * (visc_sps * xy);
+    tp[2] = one_rho * (visc_sps * xz);
+    tp[3] = one_rho * (two * yy + sumsps);
+    tp[4] = one_rho * (visc_sps * yz);
+    tp[5] = one_rho * (two * zz + sumsps);
+    if (nu_out) nu_out[p] = visc_sps;
+  });
 }
 
 // ---------------------------------------------------------------- training data
@@ -555,8 +627,9 @@ int dsph_mlp_forward(dsph_ctx* ctx, const dsph_mlp* m, uint32_t n, const float* 
                "dsph_mlp_forward: null argument");
   const unsigned ntiles = (n + 15) / 16;
   KTimer kt(ctx, "k_mlp_forward");
-  k_mlp_forward<<<std::min(ntiles, 8192u), 64, 0, ctx->stream>>>(n, d_features, m->d_wbf16,
-                                                                 m->d_params, make_norm(m), d_out);
+  const auto kernel = ntiles <= kFwdWaves ? k_mlp_forward<1> : k_mlp_forward<4>;
+  kernel<<<std::min(ntiles, kFwdWaves), 64, 0, ctx->stream>>>(n, d_features, m->d_wbf16,
+                                                              m->d_params, make_norm(m), d_out);
   DSPH_LAUNCHED(ctx, "k_mlp_forward");
   return DSPH_OK;
 }
@@ -607,7 +680,8 @@ int dsph_sps_tau_learned(dsph_ctx* ctx, const dsph_mlp* m, uint32_t np, uint32_t
                "dsph_sps_tau_learned: null argument");
   const unsigned n = np - npb, ntiles = (n + 15) / 16;
   KTimer kt(ctx, "k_sps_tau_learned");
-  k_sps_tau_learned<<<std::min(ntiles, 8192u), 64, 0, ctx->stream>>>(
+  const auto kernel = ntiles <= kFwdWaves ? k_sps_tau_learned<1> : k_sps_tau_learned<4>;
+  kernel<<<std::min(ntiles, kFwdWaves), 64, 0, ctx->stream>>>(
       n, npb, blin, dp, (const float4*)d_velrho, d_velgrad, d_sps2strain, m->d_wbf16,
       m->d_params, make_norm(m), d_tau, d_nu);
   DSPH_LAUNCHED(ctx, "k_sps_tau_learned");

@@ -56,6 +56,22 @@ def test_forward_matches_oracle(lib, ctx, n):
         net.free()
 
 
+@pytest.mark.parametrize("n", [15, 17, 65535, 65537, 65600])
+def test_forward_tile_edges(lib, ctx, n):
+    """Around one tile and around the change from one tile per wave and turn to
+    four (4096 tiles), bounds of test_forward_matches_oracle."""
+    from oracle import mlp
+    feats = _features(max(n, 64), seed=n)[:n]
+    net, p, mean, scale = _net(lib, ctx, _features(4096))
+    try:
+        got = net.forward(feats)
+        exp, _ = mlp.forward(p, feats, mean, scale, net.m.out_scale)
+        rel = np.abs(got - exp) / np.abs(exp)
+        assert rel.max() <= 1e-2 and np.median(rel) <= 1e-3, (rel.max(), np.median(rel))
+    finally:
+        net.free()
+
+
 @pytest.mark.parametrize("n,scratch_blocks", [(1003, 1024), (5000, 7)])
 def test_gradient_matches_oracle(lib, ctx, n, scratch_blocks):
     """scratch_blocks < tiles makes each block loop over several tiles."""
