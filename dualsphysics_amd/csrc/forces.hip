@@ -7,18 +7,21 @@
 // a row in ascending sorted index, all contributions in one accumulator set;
 // distances from the cell-relative FP32 PosCell.
 //
-// Two fluid kernels produce the same sums in the same order:
+// Three fluid kernels produce the same sums in the same order (fluid_form says
+// which runs):
 //  - k_forces_fluid_rows: one lane per particle looping over its rows (the
 //    reference's structure). A wave executes the pair body whenever any lane
 //    has a neighbour, so most lanes idle (about a quarter of them do work on a
 //    jittered lattice).
-//  - k_forces_fluid_tile (default): a wave walks the rows shared by its lanes
+//  - k_forces_fluid_tile: a wave walks the rows shared by its lanes
 //    once, stages each row in LDS with coalesced loads, lets every lane run a
 //    cheap conservative distance test against the staged candidates and queue
 //    its hits in LDS, then evaluates the exact pair body for the queued pairs
 //    in wave-uniform batches (every lane busy), so the expensive body runs
 //    only for real pairs. Queue order is the scan order, so the summation
 //    order is unchanged.
+//  - k_forces_fluid_team: four lanes per particle, four consecutive pairs at a
+//    time, whose terms are then added in order (small and middle sizes).
 #include <cfloat>
 #include <cstring>
 #include <map>
@@ -391,8 +394,7 @@ __global__ void __launch_bounds__(kBsForces) k_forces_fluid_rows(
 
 // Boundary particle against one fluid neighbour that passed the neighbour
 // test (KerInteractionForcesBound, JSphGpu_ker.cu:450-493): density rate and
-// the viscous dt term. Shared by the one-lane-per-particle and the tile
-// boundary kernels (same expressions, same bits).
+// the viscous dt term.
 __device__ __forceinline__ void bound_pair(const float4& vr1, const float3& dr, float rr2,
                                            const float4& vr2, float massp2, const Cte& c,
                                            float& arp1, float& visc) {
@@ -520,11 +522,8 @@ struct TileLds {
   unsigned tbase[kRing];
 };
 
-// BP1: the boundary kernel's form (KerInteractionForcesBound): p1 is a
-// boundary particle, only fluid cells are scanned, bound_pair is the pair
-// body and ar/viscdt the outputs (no neighbour pressure is needed).
 template <int TVISCO, int TDDT, bool VELGRAD, unsigned kRing, bool MDBC2 = false,
-          bool SHIFT = false, bool EOS7 = false, bool BP1 = false>
+          bool SHIFT = false, bool EOS7 = false>
 __device__ __forceinline__ void fluid_tile_body(unsigned p, bool valid, unsigned pinit,
     float viscob, float viscof, const DivData& dvd, const Cte& c, float ks2scan,
     const unsigned* __restrict__ dcell, const float4* __restrict__ poscell,
@@ -589,16 +588,10 @@ __device__ __forceinline__ void fluid_tile_body(unsigned p, bool valid, unsigned
     const unsigned jj = j & 0x7fffffffu;
     ps2 = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(poscell) + (jj << 4));
     vr2 = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(velrho) + (jj << 4));
-    if (!EOS7 && !BP1)
+    if (!EOS7)
       pr2 = *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(press) + (jj << 3));
   };
   auto eval = [&](unsigned j, const float4& ps2, const float4& vr2, const float2& pr2) {
-    if constexpr (BP1) {
-      const float3 dr = pscel_dr(q.ps, ps2, c.pcs);
-      const float rr2 = dr.x * dr.x + dr.y * dr.y + dr.z * dr.z;
-      if (rr2 <= c.ks2 && rr2 >= kAlmostZero) bound_pair(q.vr, dr, rr2, vr2, c.massf, c, a.ar, a.visc);
-      return;
-    }
     const float2 pr =
         EOS7 ? make_float2(c.cteb * (pow7_f64(vr2.w * c.ovrhopzero) - 1.0f), fast_rcp(vr2.w))
              : pr2;
@@ -653,7 +646,7 @@ __device__ __forceinline__ void fluid_tile_body(unsigned p, bool valid, unsigned
     const float qm = sqrtf(uniform_f(wave_max_f32(member ? s1 : 0.f))) + 1.01f * sqrtf(ks2scan);
     const float thr = ks2scan - s1 + 2.0e-6f * qm * qm;
     const float m2x = -2.f * q1x, m2y = -2.f * q1y, m2z = -2.f * q1z;
-    for (int kind = 0; kind < (BP1 ? 1 : 2); kind++) {
+    for (int kind = 0; kind < 2; kind++) {
       const int base = kind == 0 ? int(dvd.cellfluid) : 0;
       const unsigned kbit = unsigned(kind) << 31;
       for (int z = Z0; z < Z1; z++)
@@ -710,12 +703,7 @@ __device__ __forceinline__ void fluid_tile_body(unsigned p, bool valid, unsigned
     }
   }
   process(wave_max_u32(len), Some());
-  if (BP1) {
-    if (valid && (a.ar != 0 || a.visc != 0)) {
-      ar[p1] += a.ar;
-      if (a.visc > viscdt[p1]) viscdt[p1] = a.visc;
-    }
-  } else if (valid) {
+  if (valid) {
     store_results<TVISCO, TDDT, VELGRAD>(p1, a, viscdt, ar, ace, strain, velgrad);
     if (SHIFT) shiftposfs[p1] = a.sh;
   }
@@ -802,20 +790,730 @@ __global__ void __launch_bounds__(kBsForces) k_forces_bound(unsigned n, DivData 
   bound_body<FT>(p1, dvd, c, dcell, poscell, velrho, viscdt, ar, code, ftomassp);
 }
 
-// Boundary interaction in the tile form (same pairs, same order, same bits as
-// k_forces_bound): a wave of 64 consecutive boundary particles stages the
-// fluid rows around them in LDS and each lane tests the staged candidates.
-__global__ void __launch_bounds__(64)
-__attribute__((amdgpu_waves_per_eu(5, 8)))
-k_forces_bound_tile(unsigned n, DivData dvd, Cte c, float ks2scan,
-    const unsigned* __restrict__ dcell, const float4* __restrict__ poscell,
-    const float4* __restrict__ posf, const float4* __restrict__ velrho,
-    const float2* __restrict__ press, float* __restrict__ viscdt, float* __restrict__ ar) {
-  __shared__ TileLds<kRingTiles> lds;
-  const unsigned p = xcd_block(blockIdx.x, gridDim.x) * 64 + threadIdx.x;
-  fluid_tile_body<DSPH_VISCO_ARTIFICIAL, DSPH_DDT_NONE, false, kRingTiles, false, false, true,
-                  true>(p, p < n, 0, 0.f, 0.f, dvd, c, ks2scan, dcell, poscell, posf, velrho,
-                        press, nullptr, viscdt, ar, nullptr, nullptr, nullptr, lds);
+// Arrays of one interaction (the options' arrays are null when unused).
+struct TeamArrays {
+  const unsigned* __restrict__ dcell;
+  const float4* __restrict__ poscell;
+  const float4* __restrict__ velrho;
+  const float2* __restrict__ press;
+  const float* __restrict__ tau;
+  float* __restrict__ viscdt;
+  float* __restrict__ ar;
+  float* __restrict__ ace;
+  float* __restrict__ strain;
+  const uint8_t* __restrict__ bmode;
+  const float* __restrict__ tangenvel;
+  const typecode* __restrict__ code;
+  const float* __restrict__ ftomassp;
+};
+
+// ------------------------------------------------------------ team kernel
+// The tile kernel's sums with four lanes per particle: a wave works on 16
+// consecutive particles (a "team" of four lanes each). Rows shared by the wave's
+// particles are walked once, 64 neighbours at a time with coalesced loads; a
+// neighbour farther than 2h from the box around the particles is dropped, the
+// others go to a ring in LDS with all that the pair body reads. Every 64 of
+// them the lanes of a team test a quarter each with the conservative bound and
+// append their hits, in order, to the team's queue. The pair body then runs
+// for four consecutive hits of every team at a time, one per lane, and writes
+// the factors of its terms to LDS; each lane then adds one component (ax, ay,
+// az, ar; the density diffusion on all lanes) of the four pairs one after the other.
+// So every sum runs over the neighbours in the rows' order with the rows
+// kernel's roundings: identical bits.
+//
+// Why: with one lane per particle (tile kernel) a wave is a serial chain
+// of some 300 gathers and pair bodies, and below about 1e5 particles few
+// waves share the chip; four lanes per particle make four times the waves
+// with a quarter of the chain, and data in LDS replaces the gathers. Bound by
+// latency and VALU in about equal parts (VALU issue 77 % with 2 waves per
+// SIMD, 3 now). Dam breaks, artificial viscosity, tile -> team: 26k particles
+// 467 -> 115 us, 141k 511 -> 251 us, 357k 645 -> 573 us; boundary interaction
+// 207 -> 36, 238 -> 44 us and at 6.1M 570 -> 240 us.
+// Computed share of busy lanes in the pair body for particles in lattice order:
+// ring of 128 77 %, 192 86 %, 256 94 % (but a wave less per SIMD).
+constexpr unsigned kTeam = 4;             // lanes per particle
+constexpr unsigned kTeamP = 64 / kTeam;   // particles per wave
+constexpr unsigned kRingN = 192;          // neighbours kept in LDS (8-bit queue entries)
+constexpr unsigned kQueue = 128;          // hits a team may have queued
+constexpr int kSpan = 4;                  // cells of a row that one group spans
+constexpr int kCellBias = 128;            // cell offsets are kept as bytes
+
+template <int CTRL>
+__device__ __forceinline__ unsigned dpp_u(unsigned v) {
+  return unsigned(__builtin_amdgcn_update_dpp(0, int(v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_f(float v) {
+  return __uint_as_float(dpp_u<CTRL>(__float_as_uint(v)));
+}
+constexpr int kDppSwap1 = 0xB1;  // quad_perm [1,0,3,2]
+constexpr int kDppSwap2 = 0x4E;  // quad_perm [2,3,0,1]
+constexpr int kDppRor4 = 0x124, kDppRor8 = 0x128;  // row_ror within 16 lanes
+template <int J>
+__device__ __forceinline__ float team_lane(float v) { return dpp_f<J * 0x55>(v); }  // lane J of the team
+
+__device__ __forceinline__ void pin(float& x) { asm volatile("" : "+v"(x)); }
+__device__ __forceinline__ float lane_f(float v, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+// Minimum / maximum over the wave of a value that is equal within each team.
+__device__ __forceinline__ float teams_min(float v) {
+  v = fminf(v, dpp_f<kDppRor4>(v));
+  v = fminf(v, dpp_f<kDppRor8>(v));
+  return fminf(fminf(lane_f(v, 0), lane_f(v, 16)), fminf(lane_f(v, 32), lane_f(v, 48)));
+}
+__device__ __forceinline__ int teams_max_i(int v) {
+  v = max(v, int(dpp_u<kDppRor4>(unsigned(v))));
+  v = max(v, int(dpp_u<kDppRor8>(unsigned(v))));
+  return max(max(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+             max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
+
+// Constants of the pair body, moved to vector registers (pin): a VALU
+// instruction with a scalar register operand issues in 5 cycles on gfx950,
+// with vector registers and literals only in 2.9 (measured, v_fma_f32).
+struct PairK {
+  float pcs, ks2, invh, bwenh, eta2, mass;
+  float dk, ddtgz, rho0, pc1, pc2, pc3, pc4;  // dk = ddtkh cs0
+  float visk, h;                              // artificial: -visco cs0; else 4 visco
+  bool series;  // |ddtgz dz| < 1e-2 for every pair: the series of pow_invgamma serves all
+};
+template <int TVISCO, int TDDT>
+__device__ __forceinline__ PairK pair_k(const Cte& c, bool boundp2, float visco) {
+  PairK k;
+  k.pcs = c.pcs; k.ks2 = c.ks2; k.invh = c.invh; k.bwenh = c.bwenh; k.eta2 = c.eta2;
+  k.mass = boundp2 ? c.massb : c.massf;
+  k.dk = c.ddtkh * c.cs0; k.ddtgz = c.ddtgz; k.rho0 = c.rhopzero;
+  k.pc1 = c.pc1; k.pc2 = c.pc2; k.pc3 = c.pc3; k.pc4 = c.pc4;
+  k.visk = TVISCO == DSPH_VISCO_ARTIFICIAL ? -visco * c.cs0 : 4.f * visco;
+  k.h = c.h;
+  k.series = fabsf(c.ddtgz) * (2.f * c.h) * 1.01f < 1e-2f;
+  pin(k.pcs); pin(k.ks2); pin(k.invh); pin(k.bwenh); pin(k.eta2); pin(k.mass);
+  pin(k.visk);
+  if (TVISCO == DSPH_VISCO_ARTIFICIAL) pin(k.h);
+  if (TDDT != DSPH_DDT_NONE) pin(k.dk);
+  if (TDDT == DSPH_DDT_DDT2 || TDDT == DSPH_DDT_DDT2FULL) {
+    pin(k.ddtgz); pin(k.rho0); pin(k.pc1); pin(k.pc2); pin(k.pc3); pin(k.pc4);
+  }
+  return k;
+}
+
+// What a neighbour carries beside position, velocity, density, pressure and
+// 1/rho (only the options that use it).
+struct P2x {
+  float mass;        // FT, MDBC2: of this neighbour
+  unsigned flags;    // kNb*
+  float t[6];        // SPS: tau of a fluid neighbour; MDBC2: tangential velocity of a wall's
+};
+constexpr unsigned kNbFloating = 1, kNbLight = 2;
+
+template <int TVISCO, bool MDBC2, bool FT, bool KB>
+__device__ __forceinline__ void load_p2x(unsigned p2, const Cte& c, const TeamArrays& A, P2x& o) {
+  o.mass = 0.f;
+  o.flags = 0;
+  if (FT && !KB) {
+    o.mass = c.massf;
+    const unsigned cd = A.code[p2];
+    if (code_type(cd) == kCodeTypeFloating) {
+      const float ftm = A.ftomassp[cd & kCodeMaskValue];
+      o.flags = kNbFloating | (ftm <= c.massf * 1.2f ? kNbLight : 0u);
+      o.mass = ftm;
+    }
+  }
+  if (MDBC2 && KB) {
+    o.mass = A.bmode[p2] == DSPH_BMODE_MDBC2OFF ? 0.f : c.massb;
+#pragma unroll
+    for (int i = 0; i < 3; i++) o.t[i] = A.tangenvel[3 * size_t(p2) + i];
+  }
+  if (TVISCO == DSPH_VISCO_LAMINARSPS && !KB) {
+#pragma unroll
+    for (int i = 0; i < 6; i++) o.t[i] = A.tau[6 * size_t(p2) + i];
+  }
+}
+
+// Factors of the terms of one pair, as pair_eval adds them one after the other:
+//   a += p fr;  artificial: a += c fr, laminar: a += c dv;  SPS: a += m e,
+//   strain += u fr;  ar += mar rr;  delta -= dl.
+struct Terms {
+  float p, c, mar, dl, frx, fry, frz, rr;
+  float dvx, dvy, dvz, ex, ey, ez, m, ux, uy, uz;
+};
+
+// The terms of fluid particle q and a neighbour (pair_eval, expression by
+// expression); all zero but fr unless ok. KB: boundary neighbour.
+template <int TVISCO, int TDDT, bool MDBC2, bool FT, bool KB>
+__device__ __forceinline__ void pair_terms(bool ok, const float3& dr, float rr2, const float4& vr2,
+    float2 pr2, const P2x& x, const P1& q, const PairK& k, const Cte& c, Terms& t, float& visc,
+    bool& cancel) {
+  const float4& vr1 = q.vr;
+  const float mass = (FT && !KB) || (MDBC2 && KB) ? x.mass : k.mass;
+  const bool ftp2 = FT && !KB && (x.flags & kNbFloating);
+  const float rad = fast_sqrt(rr2);
+  const float qq = rad * k.invh;
+  const float wqq1 = 1.f - 0.5f * qq;
+  const float fac = k.bwenh * wqq1 * wqq1 * wqq1;
+  t.frx = fac * dr.x; t.fry = fac * dr.y; t.frz = fac * dr.z;
+  const float frx = t.frx, fry = t.fry, frz = t.frz;
+  const float rrho2 = pr2.y;
+  const float prs = (q.press + pr2.x) * (q.rrho * rrho2);
+  const float p = -prs * mass;
+  float dvx = vr1.x - vr2.x, dvy = vr1.y - vr2.y, dvz = vr1.z - vr2.z;
+  const float mar = mass * (dvx * frx + dvy * fry + dvz * frz);
+  const float rr = vr1.w * rrho2;
+  const float dot3 = dr.x * frx + dr.y * fry + dr.z * frz;
+  const float rr2eta = fast_rcp(rr2 + k.eta2);
+  float dl = 0.f;
+  if (TDDT == DSPH_DDT_DDT) {
+    const float rhop1over2 = vr1.w * rrho2;
+    const float visc_densi = k.dk * (rhop1over2 - 1.f) * rr2eta;
+    const float delta = visc_densi * dot3 * mass;
+    dl = -delta;
+    // A boundary neighbour cancels the term with DBC only (JSphGpu_ker.cu:665).
+    if (ok && KB && c.tboundary == DSPH_BC_DBC) cancel = true;
+    if (ok && FT && !KB && (x.flags & kNbLight)) cancel = true;
+  }
+  if (TDDT == DSPH_DDT_DDT2 && KB && ok) cancel = true;
+  if (!KB && (TDDT == DSPH_DDT_DDT2 || TDDT == DSPH_DDT_DDT2FULL)) {
+    const float rh = 1.f + k.ddtgz * dr.z;
+    const float u = rh - 1.f;
+    const float s = u * (k.pc1 + u * (k.pc2 + u * (k.pc3 + u * k.pc4)));
+    float pw = 1.f + s;
+    if (!k.series && !(fabsf(u) < 1e-2f)) pw = powf(rh, c.invgamma);
+    const float drho = k.rho0 * pw - k.rho0;
+    const float visc_densi = k.dk * ((vr2.w - vr1.w) - drho) * rr2eta;
+    const float delta = visc_densi * dot3 * mass * rrho2;
+    dl = ftp2 ? 0.f : delta;
+  }
+  if (MDBC2 && KB) {
+    dvx = vr1.x - x.t[0]; dvy = vr1.y - x.t[1]; dvz = vr1.z - x.t[2];
+  }
+  const float dot = dr.x * dvx + dr.y * dvy + dr.z * dvz;
+  const float dot_rr2 = dot * rr2eta;
+  float cc;
+  if (TVISCO == DSPH_VISCO_ARTIFICIAL) {
+    const float amubar = k.h * dot_rr2;
+    const float robar = (vr1.w + vr2.w) * 0.5f;
+    const float pi_visc = fast_div(k.visk * amubar, robar) * mass;
+    cc = dot < 0 ? -pi_visc : 0.f;
+  } else {
+    const float robar2 = (vr1.w + vr2.w);
+    const float temp = fast_div(k.visk, (rr2 + k.eta2) * robar2);
+    cc = mass * temp * dot3;
+  }
+  const unsigned keep = ok ? 0xffffffffu : 0u;
+  auto only = [&](float v) { return __uint_as_float(__float_as_uint(v) & keep); };
+  visc = fmaxf(ok ? dot_rr2 : visc, visc);
+  t.p = only(p); t.c = only(cc); t.mar = only(mar); t.dl = only(dl); t.rr = only(rr);
+  if (TVISCO != DSPH_VISCO_ARTIFICIAL) { t.dvx = only(dvx); t.dvy = only(dvy); t.dvz = only(dvz); }
+  if (TVISCO == DSPH_VISCO_LAMINARSPS) {
+    float sxx = q.tau[0], sxy = q.tau[1], sxz = q.tau[2], syy = q.tau[3], syz = q.tau[4],
+          szz = q.tau[5];
+    if (!KB && !ftp2) {
+      sxx += x.t[0]; sxy += x.t[1]; sxz += x.t[2]; syy += x.t[3]; syz += x.t[4]; szz += x.t[5];
+    }
+    t.m = only(mass);
+    t.ex = only(sxx * frx + sxy * fry + sxz * frz);
+    t.ey = only(sxy * frx + syy * fry + syz * frz);
+    t.ez = only(sxz * frx + syz * fry + szz * frz);
+    const float volp2 = -mass * rrho2;
+    const bool strain = !(FT && q.ftp1);
+    t.ux = strain ? only(dvx * volp2) : 0.f;
+    t.uy = strain ? only(dvy * volp2) : 0.f;
+    t.uz = strain ? only(dvz * volp2) : 0.f;
+  }
+}
+
+// LDS of one wave. kP: pressures; kX: floats of option data per neighbour; kM:
+// its mass; kT: float4 of terms per lane.
+template <bool kP, unsigned kX, bool kM, unsigned kT>
+struct TeamLds {
+  float4 pos[kRingN];   // PosCell position, bytes {cell offsets x, y, z, flags}
+  float4 vr[kRingN];    // velocity and density
+  float pr[kP ? kRingN : 1];    // pressure
+  float m[kM ? kRingN : 1];
+  float x[kX ? kX * kRingN : 1];
+  float4 scan[2 * 4 * 17];      // position in the group's frame, its square (17: bank spread)
+  float4 term[kTeamP * (kT * kTeam + 1)];   // a team's records, padded: bank spread
+  alignas(4) uint8_t queue[kTeamP][kQueue + 4];   // (+ 4: bank spread)
+};
+template <int TVISCO, bool MDBC2>
+constexpr unsigned team_kx() {
+  return TVISCO == DSPH_VISCO_LAMINARSPS ? 6 : (MDBC2 ? 3 : 0);
+}
+template <int TVISCO, bool BP1>
+constexpr unsigned team_kt() {
+  return BP1 ? 1 : (TVISCO == DSPH_VISCO_ARTIFICIAL ? 2 : (TVISCO == DSPH_VISCO_LAMINAR ? 3 : 5));
+}
+
+// Particles [pw, min(pw+16, n)) of those from pinit on. BP1: boundary
+// particles (bound_pair over fluid cells).
+template <int TVISCO, int TDDT, bool MDBC2, bool FT, bool BP1>
+__device__ __forceinline__ void team_body(unsigned pw, unsigned n, unsigned pinit, float viscob,
+    float viscof, const DivData& dvd, const Cte& c, const TeamArrays& A,
+    TeamLds<!BP1, team_kx<TVISCO, MDBC2>(), MDBC2 || FT, team_kt<TVISCO, BP1>()>& lds) {
+  constexpr unsigned kX = team_kx<TVISCO, MDBC2>();
+  constexpr bool kM = MDBC2 || FT;
+  constexpr bool kSps = TVISCO == DSPH_VISCO_LAMINARSPS;
+  const unsigned lane = threadIdx.x & 63u;
+  const unsigned k = lane & (kTeam - 1), team = lane / kTeam;
+  const unsigned p = pw + team;
+  const bool valid = p < n;
+  const unsigned p1 = (valid ? p : 0) + pinit;
+  P1 q;
+  q.ps = A.poscell[p1];
+  q.vr = A.velrho[p1];
+  q.press = q.rrho = 0.f;
+  if (!BP1) {
+    const float2 pr1 = A.press[p1];
+    q.press = pr1.x;
+    q.rrho = pr1.y;
+  }
+  q.ftp1 = FT && !BP1 && code_type(A.code[p1]) == kCodeTypeFloating;
+#pragma unroll
+  for (int i = 0; i < 6; i++) q.tau[i] = kSps ? A.tau[6 * size_t(p1) + i] : 0.f;
+  // This lane's sums: component k of {ax, ay, az, ar}, the diffusion, the
+  // largest dot_rr2 of its pairs, strain diagonal k and off-diagonal k
+  // (xy, xz, yz).
+  float s = 0.f, delta = 0.f, visc = 0.f, sd = 0.f, so = 0.f;
+  bool cancel = q.ftp1;
+  int cx, cy, cz;
+  {
+    const unsigned cel = A.dcell[p1];
+    cx = int(dcel_cellx(dvd.domcellcode, cel)) - dvd.czx;
+    cy = int(dcel_celly(dvd.domcellcode, cel)) - dvd.czy;
+    cz = int(dcel_cellz(dvd.domcellcode, cel)) - dvd.czz;
+  }
+  const int pfx = pscel_fx(q.ps.w), pfy = pscel_fy(q.ps.w), pfz = pscel_fz(q.ps.w);
+  const int sc = dvd.scelldiv;
+  float f1x = 0, f1y = 0, f1z = 0;  // own cell offsets from the group's, biased
+
+  // Neighbours are numbered as they are appended: [tail, scanned) tested and in
+  // the ring, [scanned, head) in the ring only (uniform). Queue of the team:
+  // qh taken, qn appended, qe[b] appended up to the end of the b-th block of
+  // 64 from tail on.
+  unsigned head = 0, scanned = 0, tail = 0;
+  unsigned qh = 0, qn = 0, qe[3] = {0, 0, 0};
+  uint8_t* const queue = lds.queue[team];
+  const unsigned kf = k < 3 ? 0xffffffffu : 0u;
+  const float* const term = reinterpret_cast<const float*>(lds.term);
+  constexpr unsigned kRec = 4 * team_kt<TVISCO, BP1>();   // floats per record
+  const unsigned tbase = team * (kTeam * kRec + 4);
+
+  // Records of the last round, added during the next one: their way through LDS
+  // and the chain of additions are covered by the pair body.
+  struct Rec { float2 ac[4]; float f[4], d[4], e[4], m[4], uk[4], ua[4], ub[4], fa[4], fb[4]; };
+  float dlp = 0.f;   // this lane's diffusion term of the last round
+  auto read = [&](Rec& v) {
+#pragma unroll
+    for (unsigned j = 0; j < kTeam; j++) {
+      const float* const r = term + tbase + j * kRec;
+      v.ac[j] = *reinterpret_cast<const float2*>(r + (BP1 || k < 3 ? 0 : 2));
+      if (BP1) continue;
+      v.f[j] = r[4 + k];
+      if (TVISCO != DSPH_VISCO_ARTIFICIAL) v.d[j] = r[8 + k];
+      if (kSps) {
+        const unsigned ia = k < 2 ? 0 : 1, ib = k == 0 ? 1 : 2;
+        v.e[j] = r[12 + k]; v.m[j] = r[19]; v.uk[j] = r[16 + k];
+        v.ua[j] = r[16 + ia]; v.ub[j] = r[16 + ib]; v.fa[j] = r[4 + ia]; v.fb[j] = r[4 + ib];
+      }
+    }
+  };
+  auto add = [&](const Rec& v) {
+    const float dl[4] = {team_lane<0>(dlp), team_lane<1>(dlp), team_lane<2>(dlp),
+                         team_lane<3>(dlp)};
+#pragma unroll
+    for (unsigned j = 0; j < kTeam; j++) {
+      s += v.ac[j].x * (BP1 ? v.ac[j].y : v.f[j]);
+      if (BP1) continue;
+      if (TVISCO == DSPH_VISCO_ARTIFICIAL)
+        s += v.ac[j].y * __uint_as_float(__float_as_uint(v.f[j]) & kf);
+      else
+        s += v.ac[j].y * v.d[j];
+      if (kSps) {
+        s += v.m[j] * v.e[j];
+        // Strain: diagonal u_k fr_k, off-diagonals xy, xz, yz.
+        sd += __uint_as_float(__float_as_uint(v.uk[j]) & kf) * v.f[j];
+        so += v.ua[j] * v.fb[j];
+        so += v.ub[j] * v.fa[j];
+      }
+      if (TDDT != DSPH_DDT_NONE) delta = delta - dl[j];
+    }
+  };
+
+  struct Nb { float4 ps, vr; float pr; P2x x; bool has; };
+  // its rounds of four consecutive hits per team.
+  auto process = [&](auto kb, const PairK& pk, int its) {
+    constexpr bool KB = decltype(kb)::value;
+    auto fetch = [&](Nb& b) {
+      const unsigned i = qh + k;
+      b.has = int(qn - i) > 0;
+      const unsigned e = queue[i & (kQueue - 1)];
+      qh = min(qh + kTeam, qn);
+      b.ps = lds.pos[e];
+      b.vr = lds.vr[e];
+      if (!BP1) b.pr = lds.pr[e];
+      if (kM) b.x.mass = lds.m[e];
+      constexpr unsigned kNx = kSps && !KB ? 6u : (MDBC2 && KB ? 3u : 0u);
+#pragma unroll
+      for (unsigned j = 0; j < kNx; j++) b.x.t[j] = lds.x[kX * e + j];
+    };
+    auto eval = [&](Nb& b) {
+      const unsigned w = __float_as_uint(b.ps.w);
+      b.x.flags = w >> 24;
+      float3 dr;
+      dr.x = q.ps.x - b.ps.x + pk.pcs * (f1x - float(w & 0xffu));
+      dr.y = q.ps.y - b.ps.y + pk.pcs * (f1y - float((w >> 8) & 0xffu));
+      dr.z = q.ps.z - b.ps.z + pk.pcs * (f1z - float((w >> 16) & 0xffu));
+      const float rr2 = dr.x * dr.x + dr.y * dr.y + dr.z * dr.z;
+      const bool ok = b.has && rr2 <= pk.ks2 && rr2 >= kAlmostZero;
+      float* const rec = reinterpret_cast<float*>(lds.term) + tbase + k * kRec;
+      Rec r;
+      read(r);
+      wave_sync();
+      if constexpr (BP1) {
+        const float mass = FT ? b.x.mass : pk.mass;
+        const float rad = fast_sqrt(rr2);
+        const float qq = rad * pk.invh;
+        const float wqq1 = 1.f - 0.5f * qq;
+        const float fac = pk.bwenh * wqq1 * wqq1 * wqq1;
+        const float frx = fac * dr.x, fry = fac * dr.y, frz = fac * dr.z;
+        const float dvx = q.vr.x - b.vr.x, dvy = q.vr.y - b.vr.y, dvz = q.vr.z - b.vr.z;
+        const float mar = mass * (dvx * frx + dvy * fry + dvz * frz);
+        const float rr = fast_div(q.vr.w, b.vr.w);
+        const float dot = dr.x * dvx + dr.y * dvy + dr.z * dvz;
+        const float dot_rr2 = fast_div(dot, rr2 + pk.eta2);
+        visc = fmaxf(ok ? dot_rr2 : visc, visc);
+        add(r);
+        *reinterpret_cast<float2*>(rec) = make_float2(ok ? mar : 0.f, ok ? rr : 0.f);
+      } else {
+        Terms t;
+        pair_terms<TVISCO, TDDT, MDBC2, FT, KB>(ok, dr, rr2, b.vr,
+                                                make_float2(b.pr, fast_rcp(b.vr.w)), b.x, q, pk, c,
+                                                t, visc, cancel);
+        add(r);
+        dlp = t.dl;
+        float4* const rec4 = reinterpret_cast<float4*>(rec);
+        // Lane 3 takes the density rate: no second factor for it.
+        rec4[0] = make_float4(t.p, t.c, t.mar, 0.f);
+        rec4[1] = make_float4(t.frx, t.fry, t.frz, t.rr);
+        if (TVISCO != DSPH_VISCO_ARTIFICIAL) rec4[2] = make_float4(t.dvx, t.dvy, t.dvz, 0.f);
+        if (kSps) {
+          rec4[3] = make_float4(t.ex, t.ey, t.ez, 0.f);
+          rec4[4] = make_float4(t.ux, t.uy, t.uz, t.m);
+        }
+      }
+      wave_sync();
+    };
+    if (its <= 0) return;
+    Nb u, v;
+    fetch(u);
+    for (;;) {
+      if (--its > 0) fetch(v);
+      eval(u);
+      if (its <= 0) break;
+      if (--its > 0) fetch(u);
+      eval(v);
+      if (its <= 0) break;
+    }
+  };
+  // Tests nb <= 64 neighbours from scanned on and queues the hits.
+  auto scan = [&](unsigned nb, bool member, float m2x, float m2y, float m2z, float thr) {
+    wave_sync();
+    const float4* const f0 = lds.scan + (scanned & 64u ? 68u : 0u) + 17 * k;
+    unsigned bits = 0;
+#pragma unroll
+    for (unsigned j = 0; j < 16; j++) {
+      const float4 f = f0[j];
+      float d = fmaf(m2x, f.x, f.w);
+      d = fmaf(m2y, f.y, d);
+      d = fmaf(m2z, f.z, d);
+      shift_in_le(bits, d, thr);
+    }
+    // Neighbour 16 k + j is at bit 15 - j.
+    bits = __builtin_bitreverse32(bits) >> 16;
+    const int nk = min(max(int(nb) - int(16 * k), 0), 16);
+    bits = member ? bits & ((1u << nk) - 1u) : 0u;
+    const unsigned a = unsigned(__popc(bits));
+    const unsigned b1 = dpp_u<kDppSwap1>(a), pair = a + b1, pair2 = dpp_u<kDppSwap2>(pair);
+    unsigned w = qn + (k & 1 ? b1 : 0u) + (k & 2 ? pair2 : 0u);
+    qn += pair + pair2;
+    const unsigned e0 = scanned % kRingN + 16 * k;
+    while (__ballot(bits != 0)) {
+      if (bits) {
+        queue[w & (kQueue - 1)] = uint8_t(e0 + unsigned(__builtin_ctz(bits)));
+        bits &= bits - 1u;
+        w++;
+      }
+    }
+    const unsigned blk = (scanned - tail) / 64;
+#pragma unroll
+    for (unsigned j = 0; j < 3; j++) qe[j] = blk == j ? qn : qe[j];
+    scanned += nb;
+    wave_sync();
+  };
+
+  // A lane without a hit reads some entry of the queue and the neighbour it names,
+  // whose contents do not count but for a finite position (the kernel gradient
+  // is not masked): entries name places of the ring and positions are finite
+  // from the start (neighbours with a position that is not fail the box test).
+  static_assert(sizeof(lds.queue) % 4 == 0, "the queues are cleared word by word");
+  for (unsigned i = lane; i < sizeof(lds.queue) / 4; i += 64)
+    reinterpret_cast<unsigned*>(lds.queue)[i] = 0u;
+  for (unsigned i = lane; i < kRingN; i += 64) lds.pos[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (unsigned i = 0; i < kRec; i++) reinterpret_cast<float*>(lds.term)[tbase + k * kRec + i] = 0.f;
+  wave_sync();
+
+  bool pending = valid;
+  for (;;) {
+    const unsigned long long pend = __ballot(pending);
+    if (!pend) break;
+    const int leader = __builtin_ctzll(pend);
+    const int gx = __builtin_amdgcn_readlane(cx, leader), gy = __builtin_amdgcn_readlane(cy, leader),
+              gz = __builtin_amdgcn_readlane(cz, leader);
+    const int rfx = __builtin_amdgcn_readlane(pfx, leader), rfy = __builtin_amdgcn_readlane(pfy, leader),
+              rfz = __builtin_amdgcn_readlane(pfz, leader);
+    const bool member = pending && cy == gy && cz == gz && unsigned(cx - gx) < unsigned(kSpan);
+    pending = pending && !member;
+    const int gxmax = gx + int(-teams_min(member ? -float(cx - gx) : 0.f));
+    const int X0 = gx - min(gx, sc), X1 = gxmax + min(dvd.ncx - gxmax - 1, sc) + 1;
+    const int Y0 = gy - min(gy, sc), Y1 = gy + min(dvd.ncy - gy - 1, sc) + 1;
+    const int Z0 = gz - min(gz, sc), Z1 = gz + min(dvd.ncz - gz - 1, sc) + 1;
+    // Positions relative to the leader's PosCell, the box of the group's
+    // particles, and the lane's threshold of the expanded distance test
+    // |q1|^2 + |q2|^2 - 2 q1.q2 <= thr (q relative to the box centre).
+    // Rounding: coordinates are below 2^4 cells, so a distance is off by less
+    // than 2^-18 cells, covered by the 4e-5 of the box test and of thr; the
+    // expanded form by 8 * 2^-24 * (2Q)^2 with Q = max|q1| + 2h.
+    if (member) {
+      f1x = float(pfx - rfx + kCellBias);
+      f1y = float(pfy - rfy + kCellBias);
+      f1z = float(pfz - rfz + kCellBias);
+    }
+    const float q1x = c.pcs * float(pfx - rfx) + q.ps.x, q1y = c.pcs * float(pfy - rfy) + q.ps.y,
+                q1z = c.pcs * float(pfz - rfz) + q.ps.z;
+    const float bx0 = teams_min(member ? q1x : FLT_MAX), bx1 = -teams_min(member ? -q1x : FLT_MAX);
+    const float by0 = teams_min(member ? q1y : FLT_MAX), by1 = -teams_min(member ? -q1y : FLT_MAX);
+    const float bz0 = teams_min(member ? q1z : FLT_MAX), bz1 = -teams_min(member ? -q1z : FLT_MAX);
+    float ox = 0.5f * (bx0 + bx1), oy = 0.5f * (by0 + by1), oz = 0.5f * (bz0 + bz1);
+    float ex = 0.5f * (bx1 - bx0), ey = 0.5f * (by1 - by0), ez = 0.5f * (bz1 - bz0);
+    float box2 = c.ks2 * 1.00004f, pcs = c.pcs;
+    pin(ox); pin(oy); pin(oz); pin(ex); pin(ey); pin(ez); pin(box2); pin(pcs);
+    const float qx = q1x - ox, qy = q1y - oy, qz = q1z - oz;
+    const float s1 = qx * qx + qy * qy + qz * qz;
+    const float qm = sqrtf(ex * ex + ey * ey + ez * ez) + 1.01f * sqrtf(c.ks2);
+    const float thr = c.ks2 * 1.00004f - s1 + 2.0e-6f * qm * qm;
+    const float m2x = -2.f * qx, m2y = -2.f * qy, m2z = -2.f * qz;
+    const int ny = Y1 - Y0, nrows = ny * (Z1 - Z0);
+
+    auto kind = [&](auto kb) {
+      constexpr bool KB = decltype(kb)::value;
+      const PairK pk = pair_k<TVISCO, TDDT>(c, KB, KB ? viscob : viscof);
+      // Rows r0.. of the group, one a lane (9 in all, or 25 of half cells).
+      int r0 = 0;
+      unsigned rini = 0, rfin = 0;
+      unsigned long long rows = 0;
+      auto load_rows = [&]() {
+        const int r = r0 + int(lane);
+        rini = rfin = 0;
+        if (r < nrows) {
+          const int z = Z0 + r / ny, y = Y0 + r % ny;
+          const int2* bc =
+              dvd.begincell + ((KB ? 0 : int(dvd.cellfluid)) + z * dvd.ncw + y * dvd.ncx);
+          for (int cl = X0; cl < X1; cl += 4) {   // row_range, four loads at a time
+            int2 be[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) be[j] = bc[min(cl + j, X1 - 1)];
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+              if (be[j].y) {
+                if (!rfin) rini = unsigned(be[j].x);
+                rfin = unsigned(be[j].y);
+              }
+          }
+        }
+        rows = __ballot(rfin > rini);
+        r0 += 64;
+      };
+      // The next 64 to come: their positions are loaded while the current
+      // ones are worked on.
+      unsigned t = 0, gfin = 0, ni = 0;
+      float4 nps = make_float4(0, 0, 0, 0);
+      bool nin = false;
+      auto advance = [&]() {
+        if (t >= gfin) {
+          while (!rows) {
+            if (r0 >= nrows) return false;
+            load_rows();
+          }
+          const int rr = __builtin_ctzll(rows);
+          rows &= rows - 1;
+          t = unsigned(__builtin_amdgcn_readlane(int(rini), rr));
+          gfin = unsigned(__builtin_amdgcn_readlane(int(rfin), rr));
+        }
+        nin = t + lane < gfin;
+        ni = nin ? t + lane : t;
+        t += 64;
+        nps = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(A.poscell) +
+                                               (ni << 4));
+        return true;
+      };
+      bool more = advance();
+      if (!more) return;
+      bool held = false;   // 64 neighbours in registers
+      float4 ps = nps, vr = nps;
+      float pr = 0;
+      unsigned ci = 0, add = 0;
+      int dx = 0, dy = 0, dz = 0;
+      float x = 0, y = 0, z = 0, s2 = 0;
+      bool keep = false;
+      unsigned long long kept = 0;
+      for (;;) {
+        if (!held && more) {
+          const bool in = nin;
+          ps = nps;
+          ci = ni;
+          vr = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(A.velrho) +
+                                                (ci << 4));
+          if (!BP1)
+            pr = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(A.press) +
+                                                 (ci << 3));
+          more = advance();
+          // Box test.
+          dx = pscel_fx(ps.w) - rfx; dy = pscel_fy(ps.w) - rfy; dz = pscel_fz(ps.w) - rfz;
+          x = pcs * float(dx) + ps.x - ox;
+          y = pcs * float(dy) + ps.y - oy;
+          z = pcs * float(dz) + ps.z - oz;
+          const float hx = fmaxf(fabsf(x) - ex, 0.f), hy = fmaxf(fabsf(y) - ey, 0.f),
+                      hz = fmaxf(fabsf(z) - ez, 0.f);
+          s2 = x * x + y * y + z * z;
+          keep = in && hx * hx + hy * hy + hz * hz <= box2 && s2 < 1e30f;
+          kept = __ballot(keep);
+          add = unsigned(__popcll(kept));
+          held = true;
+        }
+        // Append them if the ring has room, or make room by using up its
+        // oldest block; test a block of 64 if the queues have room (64 hits at
+        // most), or make room there; at the end use up all.
+        int its = 0;
+        bool fin = false;
+        if (held && head - scanned < 64) {
+          if (head + add - tail <= kRingN) {
+            if (keep) {
+              const unsigned rank = __builtin_amdgcn_mbcnt_hi(
+                  unsigned(kept >> 32), __builtin_amdgcn_mbcnt_lo(unsigned(kept), 0));
+              const unsigned si = (head + rank) & 127u;
+              lds.scan[si + (si >> 4)] = make_float4(x, y, z, s2);
+              const unsigned i = head % kRingN + rank, e = min(i, i - kRingN);
+              P2x o;
+              load_p2x<TVISCO, MDBC2, FT, KB>(ci, c, A, o);
+              const unsigned w = (unsigned(dx + kCellBias) & 0xffu) |
+                                 ((unsigned(dy + kCellBias) & 0xffu) << 8) |
+                                 ((unsigned(dz + kCellBias) & 0xffu) << 16) | (o.flags << 24);
+              lds.pos[e] = make_float4(ps.x, ps.y, ps.z, __uint_as_float(w));
+              lds.vr[e] = vr;
+              if (!BP1) lds.pr[e] = pr;
+              if (kM) lds.m[e] = o.mass;
+              constexpr unsigned kNx = kSps && !KB ? 6u : (MDBC2 && KB ? 3u : 0u);
+#pragma unroll
+              for (unsigned j = 0; j < kNx; j++) lds.x[kX * e + j] = o.t[j];
+            }
+            head += add;
+            held = false;
+          } else {
+            its = (teams_max_i(int(qe[0] - qh)) + 3) >> 2;
+            tail += 64;
+            qe[0] = qe[1]; qe[1] = qe[2];
+          }
+        }
+        const unsigned left = head - scanned;
+        const bool end = !held && !more;
+        if (left >= 64 || (end && left)) {
+          const int over = teams_max_i(int(qn - qh)) - int(kQueue - 64);
+          if (over > 0) {
+            its = (over + 3) >> 2;
+          } else {
+            scan(min(left, 64u), member, m2x, m2y, m2z, thr);
+            // Rounds that every team of the group can fill.
+            its = -teams_max_i(member ? -int(qn - qh) : -0x7fffffff) >> 2;
+          }
+        } else if (end) {
+          its = (teams_max_i(int(qn - qh)) + 3) >> 2;
+          fin = true;
+        }
+        process(kb, pk, its);
+        if (fin) break;
+      }
+      head = scanned = tail = 0;
+    };
+    kind(std::false_type());
+    if constexpr (!BP1) kind(std::true_type());
+  }
+  {
+    Rec r;
+    read(r);
+    add(r);
+  }
+  // Lane 0 of the team gathers the sums.
+  visc = fmaxf(visc, dpp_f<kDppSwap1>(visc));
+  visc = fmaxf(visc, dpp_f<kDppSwap2>(visc));
+  if constexpr (BP1) {
+    if (valid && k == 0 && (s != 0 || visc != 0)) {
+      A.ar[p1] += s;
+      if (visc > A.viscdt[p1]) A.viscdt[p1] = visc;
+    }
+  } else {
+    unsigned can = cancel ? 1u : 0u;
+    can |= dpp_u<kDppSwap1>(can);
+    can |= dpp_u<kDppSwap2>(can);
+    Acc a;
+    acc_init(a);
+    a.ax = team_lane<0>(s); a.ay = team_lane<1>(s); a.az = team_lane<2>(s); a.ar = team_lane<3>(s);
+    a.visc = visc;
+    a.delta = can ? FLT_MAX : delta;
+    if (kSps) {
+      a.s[0] = team_lane<0>(sd); a.s[3] = team_lane<1>(sd); a.s[5] = team_lane<2>(sd);
+      a.s[1] = team_lane<0>(so); a.s[2] = team_lane<1>(so); a.s[4] = team_lane<2>(so);
+    }
+    if (valid && k == 0)
+      store_results<TVISCO, TDDT, false>(p1, a, A.viscdt, A.ar, A.ace, A.strain, nullptr);
+  }
+}
+
+// Three waves per SIMD are what the LDS of ring, queues and records allows (12
+// waves per CU; a ring of 256 with 8 of them: 12.0 ms where this takes 10.6).
+template <int TVISCO, int TDDT, bool MDBC2, bool FT>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8)))
+k_forces_fluid_team(unsigned n, unsigned pinit, float viscob, float viscof, DivData dvd, Cte c,
+                    TeamArrays A) {
+  __shared__ TeamLds<true, team_kx<TVISCO, MDBC2>(), MDBC2 || FT, team_kt<TVISCO, false>()> lds;
+  team_body<TVISCO, TDDT, MDBC2, FT, false>(xcd_block(blockIdx.x, gridDim.x) * kTeamP, n, pinit,
+                                            viscob, viscof, dvd, c, A, lds);
+}
+
+template <bool FT>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8)))
+k_forces_bound_team(unsigned n, DivData dvd, Cte c, TeamArrays A) {
+  __shared__ TeamLds<false, 0, FT, 1> lds;
+  team_body<DSPH_VISCO_ARTIFICIAL, DSPH_DDT_NONE, false, FT, true>(
+      xcd_block(blockIdx.x, gridDim.x) * kTeamP, n, 0, 0.f, 0.f, dvd, c, A, lds);
+}
+
+TeamArrays team_arrays(const dsph_inter_parms* t, const float2* press) {
+  TeamArrays A;
+  A.dcell = t->d_dcell;
+  A.poscell = (const float4*)t->d_poscell;
+  A.velrho = (const float4*)t->d_velrho;
+  A.press = press;
+  A.tau = t->d_spstaurho2;
+  A.viscdt = t->d_viscdt;
+  A.ar = t->d_ar;
+  A.ace = t->d_ace;
+  A.strain = t->d_sps2strain;
+  A.bmode = t->d_boundmode;
+  A.tangenvel = t->d_tangenvel;
+  A.code = t->d_code;
+  A.ftomassp = t->d_ftomassp;
+  return A;
 }
 
 // Radius^2 of the conservative scan test: (2h + slack)^2 where the slack
@@ -823,12 +1521,54 @@ k_forces_bound_tile(unsigned n, DivData dvd, Cte c, float ks2scan,
 // half an ulp of the largest map extent, PosCell within half an ulp of pcs).
 float scan_radius2(const dsph_ctx* ctx, const Cte&) { return dsph::ens_scan_radius2(ctx->cte); }
 
+enum class FluidForm { kTeam, kTile, kRows };
+
+// Form of the fluid interaction (all give the same bits).
+// Teams win while the chip is not full of the tile kernel's waves of 64
+// particles, the tile kernel (fewer instructions per pair, 5 waves per SIMD
+// against 3) above. Measured, us, team / tile:
+//   artificial  3-D   10k fluid particles 115 / 467,  80k 251 / 511, 234k 573 / 645,
+//                     643k 1392 / 1198
+//   laminar     3-D   80k 275 / 506, 234k 645 / 656, 643k 1575 / 1202
+//   Laminar+SPS 3-D   80k 455 / 616, 157k 781 / 685
+//   artificial  2-D (step)  120k 473 / 498, 480k 769 / 699
+//   mDBC2 (laminar, step)   122k 2036 / 2375, 372k 3927 / 3894
+// Floating bodies have no tile kernel; against rows: 92k 1020 / 2286 (step),
+// 380k 2640 / 3343. Shifting has no team kernel: which boundary neighbour
+// cancels it first decides what is summed.
+FluidForm fluid_form(const dsph_ctx* ctx, const dsph_inter_parms* t) {
+  if (ctx->forces_kernel != 0 || t->d_nopenshift) return FluidForm::kRows;
+  if (t->d_ftomassp) return FluidForm::kTeam;
+  if (t->d_boundmode && (t->d_shiftposfs || t->d_velgrad)) return FluidForm::kRows;
+  if (t->d_shiftposfs || t->d_velgrad) return FluidForm::kTile;
+  const unsigned most = t->tvisco == DSPH_VISCO_ARTIFICIAL ? 320000u
+                        : t->tvisco == DSPH_VISCO_LAMINAR  ? 240000u
+                                                           : 120000u;
+  const unsigned npf = t->np - t->npb;
+  return npf <= (ctx->cte.simulate2d ? most / 2 : most) ? FluidForm::kTeam : FluidForm::kTile;
+}
+
 template <int TVISCO, int TDDT, bool VELGRAD>
 void launch_fluid(dsph_ctx* ctx, const dsph_inter_parms* t, const DivData& dvd, const Cte& c,
                   const float2* press, const float4* posf) {
   KTimer kt(ctx, "k_forces_fluid");
   const unsigned npf = t->np - t->npb;
-  if (t->d_nopenshift) {
+  const FluidForm form = fluid_form(ctx, t);
+  if (form == FluidForm::kTeam) {
+    if constexpr (!VELGRAD) {
+      const unsigned g = grid_for(npf, kTeamP);
+      const TeamArrays A = team_arrays(t, press);
+      if (t->d_ftomassp)
+        k_forces_fluid_team<TVISCO, TDDT, false, true><<<g, 64, 0, ctx->stream>>>(
+            npf, t->npb, t->viscob, t->viscof, dvd, c, A);
+      else if (t->d_boundmode)
+        k_forces_fluid_team<TVISCO, TDDT, true, false><<<g, 64, 0, ctx->stream>>>(
+            npf, t->npb, t->viscob, t->viscof, dvd, c, A);
+      else
+        k_forces_fluid_team<TVISCO, TDDT, false, false><<<g, 64, 0, ctx->stream>>>(
+            npf, t->npb, t->viscob, t->viscof, dvd, c, A);
+    }
+  } else if (t->d_nopenshift) {
     // mDBC2 with no penetration: the one-lane-per-particle kernel with the
     // no-penetration sums (shifting and floating bodies are refused with it
     // by dsph_interaction_forces).
@@ -839,8 +1579,7 @@ void launch_fluid(dsph_ctx* ctx, const dsph_inter_parms* t, const DivData& dvd, 
             t->d_sps2strain, t->d_velgrad, t->d_boundmode, t->d_tangenvel, 0, nullptr, nullptr,
             nullptr, t->d_boundnor, (float4*)t->d_nopenshift, t->d_motionvel);
   } else if (t->d_ftomassp) {
-    // Floating bodies: the one-lane-per-particle kernel with the floating
-    // rules (shifting, mDBC2 and the velocity gradient are refused with them
+    // Floating bodies, rows kernel requested (shifting, mDBC2 and the velocity gradient are refused with them
     // by dsph_interaction_forces).
     if constexpr (!VELGRAD)
       k_forces_fluid_rows<TVISCO, TDDT, false, false, false, true>
@@ -858,7 +1597,7 @@ void launch_fluid(dsph_ctx* ctx, const dsph_inter_parms* t, const DivData& dvd, 
         (const float4*)t->d_velrho, press, t->d_spstaurho2, t->d_viscdt, t->d_ar, t->d_ace,
         t->d_sps2strain, nullptr, t->d_boundmode, t->d_tangenvel, t->shiftmode, t->d_code,
         (float4*)t->d_shiftposfs);
-  } else if (t->d_shiftposfs && ctx->forces_kernel == 0) {
+  } else if (t->d_shiftposfs && form == FluidForm::kTile) {
     // Shifting in the tile kernel (no penetration and the velocity gradient
     // are refused with shifting by dsph_interaction_forces).
     k_forces_fluid_tile<TVISCO, TDDT, false, kRingTiles, false, true>
@@ -874,7 +1613,7 @@ void launch_fluid(dsph_ctx* ctx, const dsph_inter_parms* t, const DivData& dvd, 
         (const float4*)t->d_velrho, press, t->d_spstaurho2, t->d_viscdt, t->d_ar, t->d_ace,
         t->d_sps2strain, nullptr, nullptr, nullptr, t->shiftmode, t->d_code,
         (float4*)t->d_shiftposfs);
-  } else if (t->d_boundmode && ctx->forces_kernel == 0 && !VELGRAD) {
+  } else if (t->d_boundmode && form == FluidForm::kTile) {
     // mDBC2 boundaries in the tile kernel.
     k_forces_fluid_tile<TVISCO, TDDT, false, kRingTiles, true>
         <<<grid_for(npf, 64 * kTileWaves), 64 * kTileWaves, 0, ctx->stream>>>(
@@ -889,7 +1628,7 @@ void launch_fluid(dsph_ctx* ctx, const dsph_inter_parms* t, const DivData& dvd, 
         npf, t->npb, t->viscob, t->viscof, dvd, c, t->d_dcell, (const float4*)t->d_poscell,
         (const float4*)t->d_velrho, press, t->d_spstaurho2, t->d_viscdt, t->d_ar, t->d_ace,
         t->d_sps2strain, t->d_velgrad, t->d_boundmode, t->d_tangenvel);
-  } else if (ctx->forces_kernel == 0) {
+  } else if (form == FluidForm::kTile) {
     // gamma = 7 without the gradient output: the neighbour pressure is
     // evaluated in the kernel instead of being gathered (Laminar+SPS too: 127
     // registers, no spill, 9 % faster on the wave flume).
@@ -1049,25 +1788,20 @@ __global__ void __launch_bounds__(kEnsBsBoundMax) k_ens_bound(const EnsCase* __r
   bound_body<false>(ec.p0 + l, ec.dvd, ec.c, dcell, poscell, velrho, viscdt, ar);
 }
 
-// The boundary interaction of an ensemble in the tile form (k_forces_bound_tile
-// per case): bmap has one entry per 64 boundary particles.
-__global__ void __launch_bounds__(64)
-__attribute__((amdgpu_waves_per_eu(5, 8)))
-k_ens_bound_tile(const EnsCase* __restrict__ cases, const EnsState* __restrict__ st,
-    const EnsBlock* __restrict__ bmap, const unsigned* __restrict__ dcell,
-    const float4* __restrict__ poscell, const float4* __restrict__ posf,
-    const float4* __restrict__ velrho, const float2* __restrict__ press,
-    float* __restrict__ viscdt, float* __restrict__ ar) {
-  __shared__ TileLds<kRingTiles> lds;
-  const EnsBlock e = bmap[xcd_block(blockIdx.x, gridDim.x)];
+// The boundary interaction of an ensemble with teams (k_forces_bound_team per
+// case): bmap has one entry per 64 boundary particles, four waves each.
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8)))
+k_ens_bound_team(const EnsCase* __restrict__ cases, const EnsState* __restrict__ st,
+    const EnsBlock* __restrict__ bmap, TeamArrays A) {
+  __shared__ TeamLds<false, 0, false, 1> lds;
+  const unsigned b = xcd_block(blockIdx.x, gridDim.x);
+  const EnsBlock e = bmap[b / kTeam];
   if (!st[e.x].active) return;
-  const unsigned npbok = st[e.x].npbok;
-  if (e.y >= npbok) return;
+  const unsigned npbok = st[e.x].npbok, l0 = e.y + (b % kTeam) * kTeamP;
+  if (l0 >= npbok) return;
   const EnsCase& ec = cases[e.x];
-  const unsigned l = e.y + threadIdx.x;
-  fluid_tile_body<DSPH_VISCO_ARTIFICIAL, DSPH_DDT_NONE, false, kRingTiles, false, false, true,
-                  true>(l, l < npbok, ec.p0, 0.f, 0.f, ec.dvd, ec.c, ec.ks2scan, dcell, poscell,
-                        posf, velrho, press, nullptr, viscdt, ar, nullptr, nullptr, nullptr, lds);
+  team_body<DSPH_VISCO_ARTIFICIAL, DSPH_DDT_NONE, false, false, true>(l0, npbok, ec.p0, 0.f, 0.f,
+                                                                      ec.dvd, ec.c, A, lds);
 }
 
 template <int TVISCO, int TDDT, bool EOS7>
@@ -1185,13 +1919,17 @@ int ens_forces_bound(dsph_ctx* ctx, const EnsCase* cases, const EnsState* st,
 
 int ens_forces_bound_tile(dsph_ctx* ctx, const EnsCase* cases, const EnsState* st,
                           const EnsBlock* bmap64, unsigned nblocks, const unsigned* dcell,
-                          const float4* poscell, const float4* posf, const float4* velrho,
-                          const float2* press, float* viscdt, float* ar) {
+                          const float4* poscell, const float4* velrho, float* viscdt, float* ar) {
   if (!nblocks) return DSPH_OK;
   KTimer kt(ctx, "k_forces_bound");
-  k_ens_bound_tile<<<nblocks, 64, 0, ctx->stream>>>(cases, st, bmap64, dcell, poscell, posf,
-                                                    velrho, press, viscdt, ar);
-  DSPH_LAUNCHED(ctx, "k_ens_bound_tile");
+  TeamArrays A = {};
+  A.dcell = dcell;
+  A.poscell = poscell;
+  A.velrho = velrho;
+  A.viscdt = viscdt;
+  A.ar = ar;
+  k_ens_bound_team<<<nblocks * kTeam, 64, 0, ctx->stream>>>(cases, st, bmap64, A);
+  DSPH_LAUNCHED(ctx, "k_ens_bound_team");
   return DSPH_OK;
 }
 
@@ -1220,8 +1958,6 @@ int dsph_ctx_set_option(dsph_ctx* ctx, int key, int value) {
       DSPH_REQUIRE(ctx, value >= 0 && value <= 2,
                    "boundary kernel must be 0 (auto), 1 (tile) or 2 (rows)");
       ctx->bound_kernel = value;
-      ctx->bound_count = 0;
-      if (value) ctx->bound_choice = value;
       return DSPH_OK;
     default: return set_error(ctx, DSPH_E_ARG, "unknown option");
   }
@@ -1257,15 +1993,9 @@ int check_inter_parms(dsph_ctx* ctx, const dsph_inter_parms* t) {
   return DSPH_OK;
 }
 
-// Interactions between two trials of the boundary kernel's forms (auto).
-constexpr unsigned long long kBoundRetrial = 4096;
-
 // The interaction with the per-particle preparation in press/posf (np
-// entries each): k_prep, the fluid kernel, the boundary kernel. allow_trial:
-// the boundary kernel's auto choice may time its forms (events, one host
-// synchronisation per trial); without it the current choice runs.
-int interaction_forces(dsph_ctx* ctx, const dsph_inter_parms* t, float2* press, float4* posf,
-                       bool allow_trial) {
+// entries each): k_prep, the fluid kernel, the boundary kernel.
+int interaction_forces(dsph_ctx* ctx, const dsph_inter_parms* t, float2* press, float4* posf) {
   const Cte c = make_cte(ctx->cte);
   const DivData dvd = make_divdata(t->divdata);
   const unsigned npf = t->np - t->npb;
@@ -1275,7 +2005,7 @@ int interaction_forces(dsph_ctx* ctx, const dsph_inter_parms* t, float2* press, 
       KTimer kt(ctx, "k_prep");
       k_prep<<<grid_for(t->np, kBs), kBs, 0, ctx->stream>>>(
           t->np, (const float4*)t->d_poscell, (const float4*)t->d_velrho, press,
-          ctx->forces_kernel == 0 ? posf : nullptr, c);
+          fluid_form(ctx, t) == FluidForm::kTile ? posf : nullptr, c);
     }
     const bool vg = t->d_velgrad != nullptr;
     switch (t->tvisco) {
@@ -1298,47 +2028,15 @@ int interaction_forces(dsph_ctx* ctx, const dsph_inter_parms* t, float2* press, 
   }
   if (t->npbok) {
     KTimer kt(ctx, "k_forces_bound");
-    if (ctx->forces_kernel == 0 && !t->d_ftomassp && npf) {
-      // Tile or one-lane form (same pairs, same order, same bits): which is
-      // faster depends on how many walls are wet, so by default it is timed.
-      hipEvent_t* ev = nullptr;
-      int form = ctx->bound_kernel ? ctx->bound_kernel : ctx->bound_choice;
-      hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-      if (!ctx->bound_kernel && allow_trial &&
-          hipStreamIsCapturing(ctx->stream, &cs) == hipSuccess &&
-          cs == hipStreamCaptureStatusNone) {
-        // Not while a graph is being captured: the count only advances on
-        // eager interactions, so the events of a trial are always recorded.
-        const unsigned long long k = ctx->bound_count++ % kBoundRetrial;
-        if (k < 5) {
-          if (k < 4) {
-            form = k < 2 ? 1 : 2;
-            if (k == 1 || k == 3) {
-              hipEvent_t* e = ctx->bound_ev + (k == 1 ? 0 : 2);
-              for (int q = 0; q < 2; q++)
-                if (!e[q]) DSPH_HIP(ctx, hipEventCreate(&e[q]));
-              ev = e;
-            }
-          } else {
-            float ms_tile = 0, ms_rows = 0;
-            DSPH_HIP(ctx, hipEventSynchronize(ctx->bound_ev[3]));
-            DSPH_HIP(ctx, hipEventElapsedTime(&ms_tile, ctx->bound_ev[0], ctx->bound_ev[1]));
-            DSPH_HIP(ctx, hipEventElapsedTime(&ms_rows, ctx->bound_ev[2], ctx->bound_ev[3]));
-            ctx->bound_choice = ms_rows < ms_tile ? 2 : 1;
-            form = ctx->bound_choice;
-          }
-        }
-      }
-      if (ev) DSPH_HIP(ctx, hipEventRecord(ev[0], ctx->stream));
-      if (form == 1)
-        k_forces_bound_tile<<<grid_for(t->npbok, 64), 64, 0, ctx->stream>>>(
-            t->npbok, dvd, c, scan_radius2(ctx, c), t->d_dcell, (const float4*)t->d_poscell,
-            posf, (const float4*)t->d_velrho, press, t->d_viscdt, t->d_ar);
+    if (ctx->forces_kernel == 0 && ctx->bound_kernel != 2) {
+      // Teams beat one lane per particle at every size (us, dam break dp
+      // 0.02 / 0.01 / 0.0025: 36 / 44 / 240 against 207 / 238 / 350).
+      const unsigned g = grid_for(t->npbok, kTeamP);
+      const TeamArrays A = team_arrays(t, press);
+      if (t->d_ftomassp)
+        k_forces_bound_team<true><<<g, 64, 0, ctx->stream>>>(t->npbok, dvd, c, A);
       else
-        k_forces_bound<false><<<grid_for(t->npbok, kBsForces), kBsForces, 0, ctx->stream>>>(
-            t->npbok, dvd, c, t->d_dcell, (const float4*)t->d_poscell,
-            (const float4*)t->d_velrho, t->d_viscdt, t->d_ar);
-      if (ev) DSPH_HIP(ctx, hipEventRecord(ev[1], ctx->stream));
+        k_forces_bound_team<false><<<g, 64, 0, ctx->stream>>>(t->npbok, dvd, c, A);
     } else if (t->d_ftomassp)
       k_forces_bound<true><<<grid_for(t->npbok, kBsForces), kBsForces, 0, ctx->stream>>>(
           t->npbok, dvd, c, t->d_dcell, (const float4*)t->d_poscell,
@@ -1398,7 +2096,7 @@ int dsph_interaction_forces(dsph_ctx* ctx, const dsph_inter_parms* t) {
     if (rc) return rc;
   }
   return interaction_forces(ctx, t, reinterpret_cast<float2*>(ctx->prep_press),
-                            reinterpret_cast<float4*>(ctx->prep_posf), true);
+                            reinterpret_cast<float4*>(ctx->prep_posf));
 }
 
 int dsph_interaction_forces_noalloc(dsph_ctx* ctx, const dsph_inter_parms* t) {
@@ -1413,7 +2111,7 @@ int dsph_interaction_forces_noalloc(dsph_ctx* ctx, const dsph_inter_parms* t) {
     return set_error(ctx, DSPH_E_STATE, "no-alloc scratch address not set up for this device");
   unsigned char* base = static_cast<unsigned char*>(ctx->noalloc_scratch);
   return interaction_forces(ctx, t, reinterpret_cast<float2*>(base),
-                            reinterpret_cast<float4*>(base + kNoallocPressBytes), false);
+                            reinterpret_cast<float4*>(base + kNoallocPressBytes));
 }
 
 }  // extern "C"

@@ -362,12 +362,11 @@ struct dsph_ens {
     else fluid(b, bk.variant);
   }
   // Boundary interaction: s < kNumBoundBs one lane per particle in blocks
-  // of kBoundBs[s]; s == kNumBoundBs the tile form over the 64-blocks.
+  // of kBoundBs[s]; s == kNumBoundBs the form with staged neighbours over the 64-blocks.
   void bound(unsigned s) {
     if (s == kNumBoundBs)
       chk(dsph::ens_forces_bound_tile(ctx, d_cases, d_st, d_bmaps[0], nbblocks[0], dcell,
-                                      (const float4*)poscell, (const float4*)posf,
-                                      (const float4*)velrho, (const float2*)press, viscdt, ar),
+                                      (const float4*)poscell, (const float4*)velrho, viscdt, ar),
           "bound interaction");
     else
       chk(dsph::ens_forces_bound(ctx, d_cases, d_st, d_bmaps[s], nbblocks[s], kBoundBs[s],

@@ -213,16 +213,15 @@ int dsph_ctx_timing_reset(dsph_ctx* ctx);
 /* Context options (no counterpart in the reference: implementation choices
  * with identical results up to FP32 rounding). */
 #define DSPH_OPT_FORCES_KERNEL 1  /* fluid interaction kernel: 0 = cell rows
-                                     staged in LDS per wave with per-lane pair
-                                     queues (default), 1 = one lane per
-                                     particle over its cell rows */
+                                     staged in LDS per wave, four lanes or one
+                                     lane per particle by size (default), 1 =
+                                     one lane per particle over its cell rows */
 #define DSPH_OPT_BOUND_KERNEL  2  /* boundary interaction kernel (with
                                      DSPH_OPT_FORCES_KERNEL 0): 0 = auto (the
-                                     default: times both forms on interactions
-                                     1 and 3 of every 4096 and keeps the faster;
-                                     one host synchronisation per trial), 1 =
-                                     staged rows (tile), 2 = one lane per
-                                     particle. Identical bits either way. */
+                                     default, the form that is the faster at
+                                     every size: 1), 1 = staged rows, 2 = one
+                                     lane per particle. Identical bits either
+                                     way. */
 int dsph_ctx_set_option(dsph_ctx* ctx, int key, int value);
 
 /* Replaces cusph::CteInteractionUp (JSphGpu_ker.h:284). Copies into ctx. */

@@ -128,6 +128,59 @@ def test_interaction_parity(lib, ctx, name, pert, tvisco, tddt, visco, viscob, k
         assert rel_err(g["strain"][fl], o32["strain"][fl]) < TOL_FP32
 
 
+def _shuffled(c, m=None, seed=5):
+    """The first m fluid particles (all by default) moved by up to 0.15 dp,
+    with random velocities, in random order."""
+    import dataclasses
+    c = perturbed_case(c, seed=seed)
+    rng = np.random.default_rng(seed)
+    nb, m = c.nbound, c.nfluid if m is None else m
+    pos = c.pos[:nb + m].copy()
+    d = rng.uniform(-0.15 * c.dp, 0.15 * c.dp, (m, 3))
+    if c.data2d:
+        d[:, 1] = 0
+    pos[nb:] = (pos[nb:] + d)[rng.permutation(m)]
+    return dataclasses.replace(c, idp=c.idp[:nb + m], pos=pos, velrho=c.velrho[:nb + m], nfluid=m)
+
+
+_P = casemod.Parameters
+FORMS = [("n%d" % m, lambda m=m: _shuffled(casemod.dam_break(dp=0.03), m))
+         for m in (1, 15, 16, 17, 65)] + [
+    ("ddt1", lambda: _shuffled(casemod.dam_break(dp=0.02, params=_P(tdensity=N.DDT_DDT)))),
+    ("ddt2", lambda: _shuffled(casemod.dam_break(dp=0.02, params=_P(tdensity=N.DDT_DDT2)))),
+    ("laminar_half_cells", lambda: _shuffled(casemod.dam_break(
+        dp=0.02, params=_P(tvisco=N.VISCO_LAMINAR, visco=1e-4, cellmode=2)))),
+    ("sps_mdbc", lambda: _shuffled(casemod.dam_break(dp=0.02, params=_P(
+        tboundary=N.BC_MDBC, tvisco=N.VISCO_LAMINARSPS, visco=1e-6)))),
+    ("mdbc2", lambda: _shuffled(casemod.dam_break(dp=0.02, params=_P(
+        tboundary=N.BC_MDBC, slipmode=N.SLIP_NOSLIP, tvisco=N.VISCO_LAMINAR, visco=1e-4)))),
+    ("floating", lambda: casemod.dam_break_floating(dp=0.03)),
+    # Above the team kernel's sizes: the tile kernel.
+    ("tile_2d", lambda: _shuffled(casemod.dam_break_2d(dp=0.0008))),
+]
+
+
+@pytest.mark.parametrize("make", [f for _, f in FORMS], ids=[n for n, _ in FORMS])
+def test_fluid_kernel_forms_equal_bitwise(make):
+    """The form that the size and options choose (teams of lanes or the tile
+    kernel) and the rows kernel add the same terms in the same order: identical
+    bits, also around the 16 particles of a wave and for particles in no
+    order."""
+    from dualsphysics_amd.sim import SphGpuSingle
+    out = []
+    for k in (N.FORCES_TILE, N.FORCES_ROWS):   # a run of its own each: SPS keeps tau
+        s = SphGpuSingle(make())
+        try:
+            assert s.lib.dsph_ctx_set_option(s.lib.dsph_sim_ctx(s._h), N.OPT_FORCES_KERNEL, k) == 0
+            s.run(2, sync_dt=True)
+            out.append(s.forces())
+        finally:
+            s.close()
+    for a, b in zip(*out):
+        assert np.abs(b).max() > 0
+        np.testing.assert_array_equal(a, b)
+
+
 def test_tile_kernel_equals_rows_kernel_bitwise(lib, ctx):
     """Both fluid kernels sum the same pairs in the same order: identical bits."""
     c = perturbed_case(casemod.dam_break(dp=0.01), seed=3)
