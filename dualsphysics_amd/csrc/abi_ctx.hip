@@ -79,7 +79,6 @@ int dsph_ctx_destroy(dsph_ctx* ctx) {
   hipFree(ctx->sort_buf);
   hipFree(ctx->redu);
   hipFree(ctx->prep_press);
-  hipFree(ctx->prep_posf);
   hipFree(ctx->small_dev);
   if (ctx->pinned) hipHostFree(ctx->pinned);
   if (ctx->own_stream) hipStreamDestroy(ctx->own_stream);
@@ -100,10 +99,8 @@ int dsph_ctx_reserve(dsph_ctx* ctx, uint32_t np_max, uint32_t nctt_max) {
   }
   if (np_max > ctx->prep_cap) {
     hipFree(ctx->prep_press); ctx->prep_press = nullptr;
-    hipFree(ctx->prep_posf); ctx->prep_posf = nullptr;
     ctx->prep_cap = 0;
     DSPH_HIP(ctx, hipMalloc(&ctx->prep_press, 2 * sizeof(float) * size_t(np_max)));
-    DSPH_HIP(ctx, hipMalloc(&ctx->prep_posf, 4 * sizeof(float) * size_t(np_max)));
     ctx->prep_cap = np_max;
   }
   const size_t rw = (size_t(np_max) + 255) / 256 + 256;

@@ -39,7 +39,7 @@ struct EnsCase {
   PosCte pc;
   double posminx, posminy, posminz;  // PosCell map origin (Map_PosMin)
   float gx, gy, gz;     // gravity
-  float rhopoutmin, rhopoutmax, viscob, viscof, ks2scan;
+  float rhopoutmin, rhopoutmax, viscob, viscof;
   double kernelh, cs0, cfl, dtmin, tend;
   unsigned p0, np0, npb;  // first particle, particles, boundary particles
   unsigned key0, nct;     // first sort key (begincell offset), cells of the grid
@@ -87,8 +87,7 @@ struct EnsPersist {
 // ---- launchers (defined in forces.hip, step.hip, celldiv.hip); all
 // asynchronous on ctx's stream, no host synchronisation.
 int ens_prep(dsph_ctx* ctx, const EnsCase* cases, const EnsState* st, const EnsBlock* pmap,
-             unsigned npblocks, const float4* poscell, const float4* velrho, float2* press,
-             float4* posf);
+             unsigned npblocks, const float4* velrho, float2* press);
 // wmap: one entry per wave of 64 fluid particles (.y = first fluid index of
 // the wave, relative to the case's first fluid particle); without `pers`
 // every variant runs one 64-lane workgroup per entry, with it the tile
@@ -98,8 +97,7 @@ int ens_prep(dsph_ctx* ctx, const EnsCase* cases, const EnsState* st, const EnsB
 int ens_forces_fluid(dsph_ctx* ctx, int variant, int tvisco, int tddt, bool eos7,
                      const EnsCase* cases, const EnsState* st, const EnsBlock* wmap,
                      unsigned nblocks, const EnsPersist* pers, const unsigned* dcell,
-                     const float4* poscell,
-                     const float4* posf, const float4* velrho, const float2* press,
+                     const float4* poscell, const float4* velrho, const float2* press,
                      float* viscdt, float* ar, float* ace);
 // Boundary interaction with neighbours staged in LDS (teams of four lanes per
 // particle; bmap64 has one entry per 64 boundary particles).
@@ -110,9 +108,6 @@ int ens_forces_bound_tile(dsph_ctx* ctx, const EnsCase* cases, const EnsState* s
 int ens_forces_bound(dsph_ctx* ctx, const EnsCase* cases, const EnsState* st,
                      const EnsBlock* bmap, unsigned nblocks, unsigned bs, const unsigned* dcell,
                      const float4* poscell, const float4* velrho, float* viscdt, float* ar);
-
-// Radius^2 of the fluid tile kernel's conservative scan test for a case.
-float ens_scan_radius2(const dsph_cte& cte);
 
 // Zeroes ace, ar, viscdt of [0, n) (fill kernel, graph safe).
 int ens_zero_forces(dsph_ctx* ctx, unsigned n, float* ace, float* ar, float* viscdt);

@@ -38,28 +38,17 @@ constexpr unsigned kBsForces = 128;
 constexpr unsigned kBs = 256;
 
 // Per-interaction preparation: pressure (EOS once per particle; each pair sees
-// the same value the reference computes per pair), the reciprocal density
-// (v_rcp_f32, as a fast-math quotient by rho computes it), and float positions
-// in the map frame for the conservative neighbour test.
-__device__ inline void prep_one(unsigned p, const Cte& c, const float4* __restrict__ poscell,
-    const float4* __restrict__ velrho, float2* __restrict__ press, float4* __restrict__ posf) {
-  const float rho = velrho[p].w;
-  press[p] = make_float2(eos_press(rho, c), fast_rcp(rho));
-  if (posf) {
-    const float4 ps = poscell[p];
-    const double pcs = c.pcs;
-    posf[p] = make_float4(float(double(pscel_fx(ps.w)) * pcs + double(ps.x)),
-                          float(double(pscel_fy(ps.w)) * pcs + double(ps.y)),
-                          float(double(pscel_fz(ps.w)) * pcs + double(ps.z)), 0.f);
-  }
+// the same value the reference computes per pair) and the reciprocal density
+// (v_rcp_f32, as a fast-math quotient by rho computes it).
+__device__ inline float2 prep_one(float rho, const Cte& c) {
+  return make_float2(eos_press(rho, c), fast_rcp(rho));
 }
 
-__global__ void __launch_bounds__(kBs) k_prep(unsigned n, const float4* __restrict__ poscell,
-    const float4* __restrict__ velrho, float2* __restrict__ press, float4* __restrict__ posf,
-    Cte c) {
+__global__ void __launch_bounds__(kBs) k_prep(unsigned n, const float4* __restrict__ velrho,
+    float2* __restrict__ press, Cte c) {
   const unsigned p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n) return;
-  prep_one(p, c, poscell, velrho, press, posf);
+  press[p] = prep_one(velrho[p].w, c);
 }
 
 // XCD-aware block order. The dispatcher sends block i to XCD i % 8; each
@@ -98,6 +87,11 @@ struct P1 {
   float tau[6];
   bool ftp1;   // floating particle (FT kernels only)
 };
+
+// Whether the series of pow_invgamma serves every pair: |ddtgz dz| < 1e-2.
+__device__ inline bool ddt_series(const Cte& c) {
+  return fabsf(c.ddtgz) * (2.f * c.h) * 1.01f < 1e-2f;
+}
 
 // Exact pair body for fluid p1 and neighbour p2 (KerInteractionForcesFluidBox,
 // JSphGpu_ker.cu:539-777, in-scope options). boundp2 selects the boundary
@@ -169,7 +163,11 @@ __device__ __forceinline__ void pair_eval(bool boundp2, unsigned p2, const float
   if ((TDDT == DSPH_DDT_DDT2 && a.delta != FLT_MAX && !(FT && ftp2)) ||
       (TDDT == DSPH_DDT_DDT2FULL && !boundp2 && !(FT && (ftp2 || a.delta == FLT_MAX)))) {
     const float rh = 1.f + c.ddtgz * dr.z;
-    const float drho = c.rhopzero * pow_invgamma(rh, c) - c.rhopzero;
+    const float u = rh - 1.f;
+    const float ser = u * (c.pc1 + u * (c.pc2 + u * (c.pc3 + u * c.pc4)));
+    float pw = 1.f + ser;
+    if (!ddt_series(c) && !(fabsf(u) < 1e-2f)) pw = powf(rh, c.invgamma);
+    const float drho = c.rhopzero * pw - c.rhopzero;
     const float visc_densi = c.ddtkh * cbar * ((vr2.w - vr1.w) - drho) * rr2eta;
     const float delta = visc_densi * dot3 * massp2 * rrho2;
     a.delta = (boundp2 ? FLT_MAX : a.delta - delta);
@@ -217,12 +215,12 @@ __device__ __forceinline__ void pair_eval(bool boundp2, unsigned p2, const float
   const float dot_rr2 = dot * rr2eta;
   a.visc = fmaxf(dot_rr2, a.visc);
   if (TVISCO == DSPH_VISCO_ARTIFICIAL) {
-    if (dot < 0) {
-      const float amubar = c.h * dot_rr2;
-      const float robar = (vr1.w + vr2.w) * 0.5f;
-      const float pi_visc = fast_div(-visco * cbar * amubar, robar) * massp2;
-      a.ax -= pi_visc * frx; a.ay -= pi_visc * fry; a.az -= pi_visc * frz;
-    }
+    // No branch: a term of zero leaves the sums as they are.
+    const float amubar = c.h * dot_rr2;
+    const float robar = (vr1.w + vr2.w) * 0.5f;
+    float pi_visc = fast_div(-visco * cbar * amubar, robar) * massp2;
+    pi_visc = dot < 0 ? pi_visc : 0.f;
+    a.ax -= pi_visc * frx; a.ay -= pi_visc * fry; a.az -= pi_visc * frz;
   } else {
     const float robar2 = (vr1.w + vr2.w);
     const float temp = fast_div(4.f * visco, (rr2 + c.eta2) * robar2);
@@ -412,7 +410,7 @@ constexpr unsigned kTile = 64;   // candidates staged in LDS per tile (one bit e
 constexpr unsigned kMinBatch = 16;
 constexpr unsigned kScanBlock = 8;  // staged candidates tested per loop trip
 #ifndef DSPH_RING_TILES
-#define DSPH_RING_TILES 12
+#define DSPH_RING_TILES 8
 #endif
 // Tiles of hit masks kept per wave (8 bytes per lane and tile).
 constexpr unsigned kRingTiles = DSPH_RING_TILES;
@@ -435,25 +433,35 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__device__ inline unsigned wave_min_u32(unsigned v) {
-  for (int off = 32; off > 0; off >>= 1) v = min(v, (unsigned)__shfl_xor((int)v, off));
-  return v;
+template <int CTRL>
+__device__ __forceinline__ unsigned dpp_u(unsigned v) {
+  return unsigned(__builtin_amdgcn_update_dpp(0, int(v), CTRL, 0xf, 0xf, true));
 }
-__device__ inline unsigned wave_max_u32(unsigned v) {
-  for (int off = 32; off > 0; off >>= 1) v = max(v, (unsigned)__shfl_xor((int)v, off));
-  return v;
+template <int CTRL>
+__device__ __forceinline__ float dpp_f(float v) {
+  return __uint_as_float(dpp_u<CTRL>(__float_as_uint(v)));
 }
-__device__ inline int wave_max_i32(int v) {
-  for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off));
-  return v;
+constexpr int kDppRor1 = 0x121, kDppRor2 = 0x122, kDppRor4 = 0x124, kDppRor8 = 0x128;  // in 16 lanes
+__device__ __forceinline__ unsigned lane_u(unsigned v, int lane) {
+  return unsigned(__builtin_amdgcn_readlane(int(v), lane));
 }
-__device__ inline float wave_max_f32(float v) {
-  for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off));
-  return v;
+__device__ __forceinline__ float lane_f(float v, int lane) {
+  return __uint_as_float(lane_u(__float_as_uint(v), lane));
 }
-__device__ inline int uniform_i(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ inline float uniform_f(float v) {
-  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+__device__ __forceinline__ unsigned wave_min_u32(unsigned v) {
+  v = min(v, dpp_u<kDppRor8>(v));
+  v = min(v, dpp_u<kDppRor4>(v));
+  v = min(v, dpp_u<kDppRor2>(v));
+  v = min(v, dpp_u<kDppRor1>(v));
+  return min(min(lane_u(v, 0), lane_u(v, 16)), min(lane_u(v, 32), lane_u(v, 48)));
+}
+__device__ __forceinline__ unsigned wave_max_u32(unsigned v) { return ~wave_min_u32(~v); }
+__device__ __forceinline__ float wave_min_f32(float v) {
+  v = fminf(v, dpp_f<kDppRor8>(v));
+  v = fminf(v, dpp_f<kDppRor4>(v));
+  v = fminf(v, dpp_f<kDppRor2>(v));
+  v = fminf(v, dpp_f<kDppRor1>(v));
+  return fminf(fminf(lane_f(v, 0), lane_f(v, 16)), fminf(lane_f(v, 32), lane_f(v, 48)));
 }
 // Shifts the result of d <= thr into bit 0 of bits (bits = 2*bits + (thr >= d)):
 // a compare into VCC and an add with carry, two instructions per candidate.
@@ -493,49 +501,44 @@ __device__ __forceinline__ unsigned long long scan_tile(const float4* tile, unsi
   return ((unsigned long long)w[1] << 32) | w[0];
 }
 
-// Bits [k0, k1) of a 64-bit mask, 0 <= k0 <= k1 <= 64.
-__device__ inline unsigned long long bit_range(unsigned k0, unsigned k1) {
-  const unsigned long long hi = k1 >= 64 ? ~0ull : ((1ull << k1) - 1ull);
-  const unsigned long long lo = k0 >= 64 ? ~0ull : ((1ull << k0) - 1ull);
-  return hi & ~lo;
-}
-
 // One wave = 64 consecutive fluid particles (sorted order). Lanes in the same
 // cell row (cy, cz) form a group (normally the whole wave); the group walks
 // the union of its lanes' neighbour rows once, fluid cells then boundary
-// cells, z-outer / y-inner (JSphGpu_ker.cu:867-896). Each row is a contiguous
-// range of sorted particles, staged in LDS 64 at a time with coalesced loads
-// (positions relative to the group origin and their squared norm). Every lane
-// tests the staged candidates (LDS broadcast) with a conservative distance
-// bound, keeps the hits inside its own index window of the row (cells
-// cx-s..cx+s) as a 64-bit mask per tile, and the masks of the last kRing
-// tiles stay in LDS. The exact pair body then runs for the queued pairs in
+// cells, z-outer / y-inner (JSphGpu_ker.cu:867-896), 64 particles at a time with
+// coalesced loads. Those within 2h of the box around the group's particles
+// (about half) are appended, in order, to a tile in LDS (position relative to
+// the box centre and its square; the particle's index beside it). Every lane
+// tests the 64 entries of a full tile (LDS broadcast) with a conservative distance
+// bound and keeps its hits as a 64-bit mask; the masks and indices of the last
+// kRing tiles stay in LDS. The exact pair body then runs for the queued pairs in
 // wave-uniform batches (every lane busy), each lane popping its hits in tile
 // and bit order, i.e. in the reference's summation order: the results equal
 // k_forces_fluid_rows bit for bit. Loads of the next pair are issued before
 // the arithmetic of the current one.
+// Bound by the VALU (1180 instructions per particle before the box test, a tenth of
+// them scanning) and the gathers. The box test halves the tiles to scan and lets a
+// ring of 8 tiles even out the lanes better than 12 tiles of whole rows did:
+// 6.1M particles 8.04 -> 7.12 ms (rings of 6 / 10 / 12: 7.38 / 7.30 / 7.32),
+// 1.6M 2.15 -> 1.88 ms, a step of 3.0M particles in 2-D 1.99 -> 1.85 ms.
 // LDS of one wave of the tile kernel.
 template <unsigned kRing>
 struct TileLds {
-  float4 tile[kTile];
+  float4 tile[2 * kTile];   // the tiles being filled: position in the group's frame, its square
   unsigned long long masks[kRing][64];
-  unsigned tbase[kRing];
+  unsigned index[kRing * kTile];   // particle of each staged neighbour | kind << 31
 };
 
 template <int TVISCO, int TDDT, bool VELGRAD, unsigned kRing, bool MDBC2 = false,
           bool SHIFT = false, bool EOS7 = false>
 __device__ __forceinline__ void fluid_tile_body(unsigned p, bool valid, unsigned pinit,
-    float viscob, float viscof, const DivData& dvd, const Cte& c, float ks2scan,
-    const unsigned* __restrict__ dcell, const float4* __restrict__ poscell,
-    const float4* __restrict__ posf, const float4* __restrict__ velrho,
+    float viscob, float viscof, const DivData& dvd, const Cte& c,
+    const unsigned* __restrict__ dcell, const float4* __restrict__ poscell, const float4* __restrict__ velrho,
     const float2* __restrict__ press, const float* __restrict__ tau, float* __restrict__ viscdt,
     float* __restrict__ ar, float* __restrict__ ace, float* __restrict__ strain,
     float* __restrict__ velgrad, TileLds<kRing>& lds, const uint8_t* __restrict__ bmode = nullptr,
     const float* __restrict__ tangenvel = nullptr, int shiftmode = 0,
     const typecode* __restrict__ code = nullptr, float4* __restrict__ shiftposfs = nullptr) {
-  float4* tile = lds.tile;
   auto& masks = lds.masks;
-  unsigned* tbase = lds.tbase;
   const unsigned lane = threadIdx.x & 63u;
   const unsigned p1 = (valid ? p : 0) + pinit;
   Acc a;
@@ -543,7 +546,6 @@ __device__ __forceinline__ void fluid_tile_body(unsigned p, bool valid, unsigned
   P1 q;
   load_p1<TVISCO>(p1, poscell, velrho, press, tau, q);
   if (SHIFT) a.sh = shiftposfs[p1];
-  const float4 pf1 = posf[p1];
   int cx, cy, cz;
   {
     const unsigned cel = dcell[p1];
@@ -552,16 +554,16 @@ __device__ __forceinline__ void fluid_tile_body(unsigned p, bool valid, unsigned
     cz = int(dcel_cellz(dvd.domcellcode, cel)) - dvd.czz;
   }
   const int s = dvd.scelldiv;
-  const int lx0 = cx - min(cx, s), lx1 = cx + min(dvd.ncx - cx - 1, s) + 1;
+  const int pfx = pscel_fx(q.ps.w), pfy = pscel_fy(q.ps.w), pfz = pscel_fz(q.ps.w);
 
   // Queue state. wt: tiles scanned (uniform). Per lane: rt = tile being
-  // consumed, cm = its remaining hits, tb = its base index | kind << 31,
+  // consumed, cm = its remaining hits, tb = its first place in index,
   // len = queued hits. Invariant: len > 0 => cm != 0; len == 0 => rt == wt.
   unsigned wt = 0, rt = 0, tb = 0, len = 0;
   unsigned long long cm = 0;
   auto pop = [&](unsigned& j) {
     const unsigned bit = unsigned(__builtin_ctzll(cm));  // cm != 0 while len > 0
-    j = tb + bit;  // kind bit 31 carried along
+    j = lds.index[tb + bit];  // kind in bit 31
     cm &= cm - 1ull;
     len--;
     if (!cm) {
@@ -570,7 +572,7 @@ __device__ __forceinline__ void fluid_tile_body(unsigned p, bool valid, unsigned
           rt++;
           cm = masks[rt % kRing][lane];
         } while (!cm);
-        tb = tbase[rt % kRing];
+        tb = rt % kRing * kTile;
       } else {
         rt = wt;
       }
@@ -627,79 +629,125 @@ __device__ __forceinline__ void fluid_tile_body(unsigned p, bool valid, unsigned
     const unsigned long long pend = __ballot(pending);
     if (!pend) break;
     const int leader = __ffsll((long long)pend) - 1;
-    const int gy = uniform_i(__shfl(cy, leader)), gz = uniform_i(__shfl(cz, leader));
+    const int gy = __builtin_amdgcn_readlane(cy, leader), gz = __builtin_amdgcn_readlane(cz, leader);
+    const int rfx = __builtin_amdgcn_readlane(pfx, leader),
+              rfy = __builtin_amdgcn_readlane(pfy, leader),
+              rfz = __builtin_amdgcn_readlane(pfz, leader);
     const bool member = pending && cy == gy && cz == gz;
     pending = pending && !member;
-    const int gxmin = uniform_i(__shfl(cx, leader));
-    const int gxmax = uniform_i(wave_max_i32(member ? cx : -1));
+    const int gxmin = __builtin_amdgcn_readlane(cx, leader);
+    const int gxmax = int(~wave_min_u32(member ? ~unsigned(cx) : 0xffffffffu));
     const int X0 = gxmin - min(gxmin, s), X1 = gxmax + min(dvd.ncx - gxmax - 1, s) + 1;
     const int Y0 = gy - min(gy, s), Y1 = gy + min(dvd.ncy - gy - 1, s) + 1;
     const int Z0 = gz - min(gz, s), Z1 = gz + min(dvd.ncz - gz - 1, s) + 1;
-    // Group origin and the per-lane threshold of the expanded distance test
-    // |q1|^2 + |q2|^2 - 2 q1.q2 <= ks2scan (q relative to the origin). For a
-    // real neighbour |q|,|q2| <= Q = max|q1| + 2h, and the rounding of the
-    // expanded form stays below 8 * 2^-24 * (2Q)^2.
-    const float ox = uniform_f(__shfl(pf1.x, leader)), oy = uniform_f(__shfl(pf1.y, leader)),
-                oz = uniform_f(__shfl(pf1.z, leader));
-    const float q1x = pf1.x - ox, q1y = pf1.y - oy, q1z = pf1.z - oz;
-    const float s1 = q1x * q1x + q1y * q1y + q1z * q1z;
-    const float qm = sqrtf(uniform_f(wave_max_f32(member ? s1 : 0.f))) + 1.01f * sqrtf(ks2scan);
-    const float thr = ks2scan - s1 + 2.0e-6f * qm * qm;
-    const float m2x = -2.f * q1x, m2y = -2.f * q1y, m2z = -2.f * q1z;
-    for (int kind = 0; kind < 2; kind++) {
-      const int base = kind == 0 ? int(dvd.cellfluid) : 0;
-      const unsigned kbit = unsigned(kind) << 31;
-      for (int z = Z0; z < Z1; z++)
-        for (int y = Y0; y < Y1; y++) {
-          const int rowbase = base + z * dvd.ncw + y * dvd.ncx;
-          unsigned gini, gfin;
-          row_range(dvd.begincell, rowbase, X0, X1, gini, gfin);
-          gini = unsigned(uniform_i(int(gini)));
-          gfin = unsigned(uniform_i(int(gfin)));
-          if (gfin <= gini) continue;
-          unsigned lo = 0, hi = 0;
-          if (member) row_range(dvd.begincell, rowbase, lx0, lx1, lo, hi);
-          for (unsigned t = gini; t < gfin; t += kTile) {
-            // The ring slot of tile wt must have been consumed by every lane.
-            while (wt >= kRing && wave_min_u32(rt) <= wt - kRing) process(kMinBatch, Some());
-            wave_sync();
-            if (t + lane < gfin) {
-              const float4 f = posf[t + lane];
-              const float x = f.x - ox, y2 = f.y - oy, z2 = f.z - oz;
-              tile[lane] = make_float4(x, y2, z2, x * x + y2 * y2 + z2 * z2);
-            }
-            if (lane == 0) tbase[wt % kRing] = t | kbit;
-            wave_sync();
-            // Hits of this lane among the staged candidates (blocks of 8 up
-            // to the last staged one; the window drops the rest).
-            unsigned long long hm = 0;
-            if (member) {
-              const unsigned k0 = lo > t ? min(lo - t, kTile) : 0u;
-              const unsigned k1 = hi > t ? min(hi - t, kTile) : 0u;
-              const unsigned long long win = k1 > k0 ? bit_range(k0, k1) : 0ull;
-              if (win) {
-                const unsigned nblk = (min(kTile, gfin - t) + kScanBlock - 1) / kScanBlock;
-                hm = scan_tile(tile, nblk, m2x, m2y, m2z, thr) & win;
-              }
-            }
-            masks[wt % kRing][lane] = hm;
-            if (len == 0) {
-              // Caught up: consume the new tile directly.
-              cm = hm;
-              tb = t | kbit;
-              rt = hm ? wt : wt + 1;
-            }
-            len += unsigned(__popcll(hm));
-            wt++;
-            const unsigned mn = wave_min_u32(member ? len : 0xffffffffu);
-            if (mn >= kMinBatch) {
-              // All 64 lanes have mn pairs queued (the usual case: one group,
-              // all lanes valid): batches without per-lane tests.
-              if (wave_min_u32(len) >= mn) process(mn, Full());
-              else process(mn, Some());
-            }
+    // Positions relative to the leader's PosCell, the box of the group's
+    // particles, and the lane's threshold of the expanded distance test
+    // |q1|^2 + |q2|^2 - 2 q1.q2 <= thr (q relative to the box centre).
+    // Rounding: of the coordinates below 2^-22 Q with Q = max|q1| + 2h, of the
+    // expanded form below 8 * 2^-24 * (2Q)^2: covered by 4e-5 (2h)^2 + 2e-6 Q^2.
+    const float q1x = c.pcs * float(pfx - rfx) + q.ps.x, q1y = c.pcs * float(pfy - rfy) + q.ps.y,
+                q1z = c.pcs * float(pfz - rfz) + q.ps.z;
+    const float bx0 = wave_min_f32(member ? q1x : FLT_MAX),
+                bx1 = -wave_min_f32(member ? -q1x : FLT_MAX);
+    const float by0 = wave_min_f32(member ? q1y : FLT_MAX),
+                by1 = -wave_min_f32(member ? -q1y : FLT_MAX);
+    const float bz0 = wave_min_f32(member ? q1z : FLT_MAX),
+                bz1 = -wave_min_f32(member ? -q1z : FLT_MAX);
+    const float ox = 0.5f * (bx0 + bx1), oy = 0.5f * (by0 + by1), oz = 0.5f * (bz0 + bz1);
+    const float ex = 0.5f * (bx1 - bx0), ey = 0.5f * (by1 - by0), ez = 0.5f * (bz1 - bz0);
+    const float qx = q1x - ox, qy = q1y - oy, qz = q1z - oz;
+    const float s1 = qx * qx + qy * qy + qz * qz;
+    const float qm = sqrtf(ex * ex + ey * ey + ez * ez) + 1.01f * sqrtf(c.ks2);
+    const float box2 = c.ks2 * 1.00004f + 2.0e-6f * qm * qm;
+    const float thr = box2 - s1;
+    const float m2x = -2.f * qx, m2y = -2.f * qy, m2z = -2.f * qz;
+    const int ny = Y1 - Y0, nrows = ny * (Z1 - Z0);
+    // Rows of the group, fluid cells then boundary cells, one a lane (18 in
+    // all, or 50 of half cells); 64 neighbours of a row at a time. Those near
+    // the group's box are appended to the tile being filled (index wt; fill
+    // entries, the ones past 64 belong to the next).
+    int r0 = 0;
+    unsigned rini = 0, rfin = 0, t = 0, gfin = 0, kbit = 0, fill = 0;
+    unsigned long long rows = 0;
+    for (bool more = true; more;) {
+      if (t >= gfin) {
+        while (!rows && r0 < 2 * nrows) {
+          const int r = r0 + int(lane);
+          rini = rfin = 0;
+          if (r < 2 * nrows) {
+            const int rk = r >= nrows ? r - nrows : r;
+            const int z = Z0 + rk / ny, y = Y0 + rk % ny;
+            row_range(dvd.begincell,
+                      (r >= nrows ? 0 : int(dvd.cellfluid)) + z * dvd.ncw + y * dvd.ncx, X0, X1,
+                      rini, rfin);
           }
+          rows = __ballot(rfin > rini);
+          r0 += 64;
         }
+        more = rows != 0;
+        if (more) {
+          const int rr = __builtin_ctzll(rows);
+          rows &= rows - 1;
+          t = lane_u(rini, rr);
+          gfin = lane_u(rfin, rr);
+          kbit = r0 - 64 + rr >= nrows ? 0x80000000u : 0u;
+        }
+      }
+      if (more) {
+        // The places of tiles wt and wt + 1 must have been consumed by every lane.
+        while (wt + 1 >= kRing && wave_min_u32(rt) + kRing <= wt + 1) process(kMinBatch, Some());
+        const bool in = t + lane < gfin;
+        const unsigned p2 = in ? t + lane : t;
+        t += 64;
+        const float4 f = *reinterpret_cast<const float4*>(
+            reinterpret_cast<const char*>(poscell) + (p2 << 4));
+        const float x = c.pcs * float(pscel_fx(f.w) - rfx) + f.x - ox,
+                    y = c.pcs * float(pscel_fy(f.w) - rfy) + f.y - oy,
+                    z = c.pcs * float(pscel_fz(f.w) - rfz) + f.z - oz;
+        const float hx = fmaxf(fabsf(x) - ex, 0.f), hy = fmaxf(fabsf(y) - ey, 0.f),
+                    hz = fmaxf(fabsf(z) - ez, 0.f);
+        const bool keep = in && hx * hx + hy * hy + hz * hz <= box2;
+        const unsigned long long kept = __ballot(keep);
+        wave_sync();
+        if (keep) {
+          const unsigned i = fill + __builtin_amdgcn_mbcnt_hi(
+                                        unsigned(kept >> 32),
+                                        __builtin_amdgcn_mbcnt_lo(unsigned(kept), 0));
+          lds.tile[(wt * kTile + i) % (2 * kTile)] = make_float4(x, y, z, x * x + y * y + z * z);
+          const unsigned e = wt % kRing * kTile + i;
+          lds.index[e >= kRing * kTile ? e - kRing * kTile : e] = p2 | kbit;
+        }
+        fill += unsigned(__popcll(kept));
+        wave_sync();
+      }
+      if (fill >= kTile || (!more && fill)) {
+        // Hits of this lane among the entries of the tile (blocks of 8 up to the
+        // last one; the rest drops).
+        const unsigned nt = min(fill, kTile);
+        unsigned long long hm = 0;
+        if (member)
+          hm = scan_tile(lds.tile + (wt & 1) * kTile, (nt + kScanBlock - 1) / kScanBlock, m2x, m2y,
+                         m2z, thr) &
+               (~0ull >> (kTile - nt));
+        masks[wt % kRing][lane] = hm;
+        if (len == 0) {
+          // Caught up: consume the new tile directly.
+          cm = hm;
+          tb = wt % kRing * kTile;
+          rt = hm ? wt : wt + 1;
+        }
+        len += unsigned(__popcll(hm));
+        wt++;
+        fill -= nt;
+        if (!more && fill) more = true;   // a last, partial tile
+        const unsigned mn = wave_min_u32(member ? len : 0xffffffffu);
+        if (mn >= kMinBatch) {
+          // All 64 lanes have mn pairs queued (the usual case: one group,
+          // all lanes valid): batches without per-lane tests.
+          if (wave_min_u32(len) >= mn) process(mn, Full());
+          else process(mn, Some());
+        }
+      }
     }
   }
   process(wave_max_u32(len), Some());
@@ -725,9 +773,8 @@ template <int TVISCO, int TDDT, bool VELGRAD, unsigned kRing, bool MDBC2 = false
 __global__ void __launch_bounds__(64 * kTileWaves)
 __attribute__((amdgpu_waves_per_eu(tile_min_waves<TVISCO, VELGRAD, MDBC2, SHIFT>(), 8)))
 k_forces_fluid_tile(
-    unsigned n, unsigned pinit, float viscob, float viscof, DivData dvd, Cte c, float ks2scan,
-    const unsigned* __restrict__ dcell, const float4* __restrict__ poscell,
-    const float4* __restrict__ posf, const float4* __restrict__ velrho,
+    unsigned n, unsigned pinit, float viscob, float viscof, DivData dvd, Cte c,
+    const unsigned* __restrict__ dcell, const float4* __restrict__ poscell, const float4* __restrict__ velrho,
     const float2* __restrict__ press, const float* __restrict__ tau, float* __restrict__ viscdt,
     float* __restrict__ ar, float* __restrict__ ace, float* __restrict__ strain,
     float* __restrict__ velgrad, const uint8_t* __restrict__ bmode = nullptr,
@@ -738,7 +785,7 @@ k_forces_fluid_tile(
   const unsigned p =
       (xcd_block(blockIdx.x, gridDim.x) * kTileWaves + w) * 64 + (threadIdx.x & 63u);
   fluid_tile_body<TVISCO, TDDT, VELGRAD, kRing, MDBC2, SHIFT, EOS7>(
-      p, p < n, pinit, viscob, viscof, dvd, c, ks2scan, dcell, poscell, posf, velrho, press, tau,
+      p, p < n, pinit, viscob, viscof, dvd, c, dcell, poscell, velrho, press, tau,
       viscdt, ar, ace, strain, velgrad, lds[w], bmode, tangenvel, shiftmode, code, shiftposfs);
 }
 
@@ -838,24 +885,12 @@ constexpr unsigned kQueue = 128;          // hits a team may have queued
 constexpr int kSpan = 4;                  // cells of a row that one group spans
 constexpr int kCellBias = 128;            // cell offsets are kept as bytes
 
-template <int CTRL>
-__device__ __forceinline__ unsigned dpp_u(unsigned v) {
-  return unsigned(__builtin_amdgcn_update_dpp(0, int(v), CTRL, 0xf, 0xf, true));
-}
-template <int CTRL>
-__device__ __forceinline__ float dpp_f(float v) {
-  return __uint_as_float(dpp_u<CTRL>(__float_as_uint(v)));
-}
 constexpr int kDppSwap1 = 0xB1;  // quad_perm [1,0,3,2]
 constexpr int kDppSwap2 = 0x4E;  // quad_perm [2,3,0,1]
-constexpr int kDppRor4 = 0x124, kDppRor8 = 0x128;  // row_ror within 16 lanes
 template <int J>
 __device__ __forceinline__ float team_lane(float v) { return dpp_f<J * 0x55>(v); }  // lane J of the team
 
 __device__ __forceinline__ void pin(float& x) { asm volatile("" : "+v"(x)); }
-__device__ __forceinline__ float lane_f(float v, int lane) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
-}
 // Minimum / maximum over the wave of a value that is equal within each team.
 __device__ __forceinline__ float teams_min(float v) {
   v = fminf(v, dpp_f<kDppRor4>(v));
@@ -887,7 +922,7 @@ __device__ __forceinline__ PairK pair_k(const Cte& c, bool boundp2, float visco)
   k.pc1 = c.pc1; k.pc2 = c.pc2; k.pc3 = c.pc3; k.pc4 = c.pc4;
   k.visk = TVISCO == DSPH_VISCO_ARTIFICIAL ? -visco * c.cs0 : 4.f * visco;
   k.h = c.h;
-  k.series = fabsf(c.ddtgz) * (2.f * c.h) * 1.01f < 1e-2f;
+  k.series = ddt_series(c);
   pin(k.pcs); pin(k.ks2); pin(k.invh); pin(k.bwenh); pin(k.eta2); pin(k.mass);
   pin(k.visk);
   if (TVISCO == DSPH_VISCO_ARTIFICIAL) pin(k.h);
@@ -1516,11 +1551,6 @@ TeamArrays team_arrays(const dsph_inter_parms* t, const float2* press) {
   return A;
 }
 
-// Radius^2 of the conservative scan test: (2h + slack)^2 where the slack
-// bounds the rounding of map-frame float positions (each coordinate within
-// half an ulp of the largest map extent, PosCell within half an ulp of pcs).
-float scan_radius2(const dsph_ctx* ctx, const Cte&) { return dsph::ens_scan_radius2(ctx->cte); }
-
 enum class FluidForm { kTeam, kTile, kRows };
 
 // Form of the fluid interaction (all give the same bits).
@@ -1550,7 +1580,7 @@ FluidForm fluid_form(const dsph_ctx* ctx, const dsph_inter_parms* t) {
 
 template <int TVISCO, int TDDT, bool VELGRAD>
 void launch_fluid(dsph_ctx* ctx, const dsph_inter_parms* t, const DivData& dvd, const Cte& c,
-                  const float2* press, const float4* posf) {
+                  const float2* press) {
   KTimer kt(ctx, "k_forces_fluid");
   const unsigned npf = t->np - t->npb;
   const FluidForm form = fluid_form(ctx, t);
@@ -1602,8 +1632,8 @@ void launch_fluid(dsph_ctx* ctx, const dsph_inter_parms* t, const DivData& dvd, 
     // are refused with shifting by dsph_interaction_forces).
     k_forces_fluid_tile<TVISCO, TDDT, false, kRingTiles, false, true>
         <<<grid_for(npf, 64 * kTileWaves), 64 * kTileWaves, 0, ctx->stream>>>(
-        npf, t->npb, t->viscob, t->viscof, dvd, c, scan_radius2(ctx, c), t->d_dcell,
-        (const float4*)t->d_poscell, posf, (const float4*)t->d_velrho, press, t->d_spstaurho2,
+        npf, t->npb, t->viscob, t->viscof, dvd, c, t->d_dcell,
+        (const float4*)t->d_poscell, (const float4*)t->d_velrho, press, t->d_spstaurho2,
         t->d_viscdt, t->d_ar, t->d_ace, t->d_sps2strain, nullptr, nullptr, nullptr, t->shiftmode,
         t->d_code, (float4*)t->d_shiftposfs);
   } else if (t->d_shiftposfs) {
@@ -1617,8 +1647,8 @@ void launch_fluid(dsph_ctx* ctx, const dsph_inter_parms* t, const DivData& dvd, 
     // mDBC2 boundaries in the tile kernel.
     k_forces_fluid_tile<TVISCO, TDDT, false, kRingTiles, true>
         <<<grid_for(npf, 64 * kTileWaves), 64 * kTileWaves, 0, ctx->stream>>>(
-        npf, t->npb, t->viscob, t->viscof, dvd, c, scan_radius2(ctx, c), t->d_dcell,
-        (const float4*)t->d_poscell, posf, (const float4*)t->d_velrho, press, t->d_spstaurho2,
+        npf, t->npb, t->viscob, t->viscof, dvd, c, t->d_dcell,
+        (const float4*)t->d_poscell, (const float4*)t->d_velrho, press, t->d_spstaurho2,
         t->d_viscdt, t->d_ar, t->d_ace, t->d_sps2strain, nullptr, t->d_boundmode, t->d_tangenvel);
   } else if (t->d_boundmode) {
     // mDBC2 with the velocity gradient (learned closure) or the rows kernel
@@ -1636,14 +1666,14 @@ void launch_fluid(dsph_ctx* ctx, const dsph_inter_parms* t, const DivData& dvd, 
     if (kEos7Built && c.gamma == 7.f)
       k_forces_fluid_tile<TVISCO, TDDT, false, kRingTiles, false, false, kEos7Built>
           <<<grid_for(npf, 64 * kTileWaves), 64 * kTileWaves, 0, ctx->stream>>>(
-              npf, t->npb, t->viscob, t->viscof, dvd, c, scan_radius2(ctx, c), t->d_dcell,
-              (const float4*)t->d_poscell, posf, (const float4*)t->d_velrho, press,
+              npf, t->npb, t->viscob, t->viscof, dvd, c, t->d_dcell,
+              (const float4*)t->d_poscell, (const float4*)t->d_velrho, press,
               t->d_spstaurho2, t->d_viscdt, t->d_ar, t->d_ace, t->d_sps2strain, nullptr);
     else
       k_forces_fluid_tile<TVISCO, TDDT, VELGRAD, kRingTiles>
           <<<grid_for(npf, 64 * kTileWaves), 64 * kTileWaves, 0, ctx->stream>>>(
-              npf, t->npb, t->viscob, t->viscof, dvd, c, scan_radius2(ctx, c), t->d_dcell,
-              (const float4*)t->d_poscell, posf, (const float4*)t->d_velrho, press,
+              npf, t->npb, t->viscob, t->viscof, dvd, c, t->d_dcell,
+              (const float4*)t->d_poscell, (const float4*)t->d_velrho, press,
               t->d_spstaurho2, t->d_viscdt, t->d_ar, t->d_ace, t->d_sps2strain, t->d_velgrad);
   } else {
     k_forces_fluid_rows<TVISCO, TDDT, VELGRAD, false><<<grid_for(npf, kBsForces), kBsForces, 0,
@@ -1656,13 +1686,13 @@ void launch_fluid(dsph_ctx* ctx, const dsph_inter_parms* t, const DivData& dvd, 
 
 template <int TVISCO, bool VELGRAD>
 int dispatch_ddt(dsph_ctx* ctx, const dsph_inter_parms* t, const DivData& dvd, const Cte& c,
-                 const float2* press, const float4* posf) {
+                 const float2* press) {
   switch (t->tdensity) {
-    case DSPH_DDT_NONE: launch_fluid<TVISCO, DSPH_DDT_NONE, VELGRAD>(ctx, t, dvd, c, press, posf); break;
-    case DSPH_DDT_DDT: launch_fluid<TVISCO, DSPH_DDT_DDT, VELGRAD>(ctx, t, dvd, c, press, posf); break;
-    case DSPH_DDT_DDT2: launch_fluid<TVISCO, DSPH_DDT_DDT2, VELGRAD>(ctx, t, dvd, c, press, posf); break;
+    case DSPH_DDT_NONE: launch_fluid<TVISCO, DSPH_DDT_NONE, VELGRAD>(ctx, t, dvd, c, press); break;
+    case DSPH_DDT_DDT: launch_fluid<TVISCO, DSPH_DDT_DDT, VELGRAD>(ctx, t, dvd, c, press); break;
+    case DSPH_DDT_DDT2: launch_fluid<TVISCO, DSPH_DDT_DDT2, VELGRAD>(ctx, t, dvd, c, press); break;
     case DSPH_DDT_DDT2FULL:
-      launch_fluid<TVISCO, DSPH_DDT_DDT2FULL, VELGRAD>(ctx, t, dvd, c, press, posf);
+      launch_fluid<TVISCO, DSPH_DDT_DDT2FULL, VELGRAD>(ctx, t, dvd, c, press);
       break;
     default: return set_error(ctx, DSPH_E_ARG, "dsph_interaction_forces: invalid tdensity");
   }
@@ -1679,14 +1709,13 @@ __global__ void k_fill_u32(unsigned* __restrict__ a, unsigned n, unsigned v) {
 
 __global__ void __launch_bounds__(kBs) k_ens_prep(const EnsCase* __restrict__ cases,
     const EnsState* __restrict__ st, const EnsBlock* __restrict__ pmap,
-    const float4* __restrict__ poscell, const float4* __restrict__ velrho,
-    float2* __restrict__ press, float4* __restrict__ posf) {
+    const float4* __restrict__ velrho, float2* __restrict__ press) {
   const EnsBlock e = pmap[blockIdx.x];
   if (!st[e.x].active) return;
   const unsigned l = e.y + threadIdx.x;
   if (l >= st[e.x].np) return;
   const EnsCase& ec = cases[e.x];
-  prep_one(ec.p0 + l, ec.c, poscell, velrho, press, posf);
+  press[ec.p0 + l] = prep_one(velrho[ec.p0 + l].w, ec.c);
 }
 
 template <int TVISCO, int TDDT, unsigned kRing, bool EOS7>
@@ -1694,8 +1723,7 @@ __global__ void __launch_bounds__(64)
 __attribute__((amdgpu_waves_per_eu(tile_min_waves<TVISCO, false, false, false>(), 8)))
 k_ens_fluid_tile(const EnsCase* __restrict__ cases,
     const EnsState* __restrict__ st, const EnsBlock* __restrict__ wmap,
-    const unsigned* __restrict__ dcell, const float4* __restrict__ poscell,
-    const float4* __restrict__ posf, const float4* __restrict__ velrho,
+    const unsigned* __restrict__ dcell, const float4* __restrict__ poscell, const float4* __restrict__ velrho,
     const float2* __restrict__ press, float* __restrict__ viscdt, float* __restrict__ ar,
     float* __restrict__ ace) {
   __shared__ TileLds<kRing> lds;
@@ -1707,7 +1735,7 @@ k_ens_fluid_tile(const EnsCase* __restrict__ cases,
   const unsigned p = e.y + threadIdx.x;
   fluid_tile_body<TVISCO, TDDT, false, kRing, false, false, EOS7>(
       p, p < npf, ec.p0 + ec.npb, ec.viscob, ec.viscof,
-                                              ec.dvd, ec.c, ec.ks2scan, dcell, poscell, posf,
+                                              ec.dvd, ec.c, dcell, poscell,
                                               velrho, press, nullptr, viscdt, ar, ace, nullptr,
                                               nullptr, lds);
 }
@@ -1727,8 +1755,7 @@ __attribute__((amdgpu_waves_per_eu(tile_min_waves<TVISCO, false, false, false>()
 k_ens_fluid_tile_persist(const EnsCase* __restrict__ cases,
     const EnsState* __restrict__ st, const EnsBlock* __restrict__ wmap, unsigned nitems,
     unsigned chunk, unsigned* __restrict__ ctr,
-    const unsigned* __restrict__ dcell, const float4* __restrict__ poscell,
-    const float4* __restrict__ posf, const float4* __restrict__ velrho,
+    const unsigned* __restrict__ dcell, const float4* __restrict__ poscell, const float4* __restrict__ velrho,
     const float2* __restrict__ press, float* __restrict__ viscdt, float* __restrict__ ar,
     float* __restrict__ ace) {
   __shared__ TileLds<kRing> lds;
@@ -1751,8 +1778,8 @@ k_ens_fluid_tile_persist(const EnsCase* __restrict__ cases,
         if (e.y >= npf) continue;
         const unsigned p = e.y + threadIdx.x;
         fluid_tile_body<TVISCO, TDDT, false, kRing, false, false, EOS7>(
-            p, p < npf, ec.p0 + ec.npb, ec.viscob, ec.viscof, ec.dvd, ec.c, ec.ks2scan, dcell,
-            poscell, posf, velrho, press, nullptr, viscdt, ar, ace, nullptr, nullptr, lds);
+            p, p < npf, ec.p0 + ec.npb, ec.viscob, ec.viscof, ec.dvd, ec.c, dcell,
+            poscell, velrho, press, nullptr, viscdt, ar, ace, nullptr, nullptr, lds);
       }
     }
   }
@@ -1808,24 +1835,24 @@ template <int TVISCO, int TDDT, bool EOS7>
 void launch_ens_fluid(dsph_ctx* ctx, int variant, const EnsCase* cases, const EnsState* st,
                       const EnsBlock* wmap, unsigned nb, const EnsPersist* pers,
                       const unsigned* dcell,
-                      const float4* poscell, const float4* posf, const float4* velrho,
+                      const float4* poscell, const float4* velrho,
                       const float2* press, float* viscdt, float* ar, float* ace) {
   if (pers) {
     const unsigned g = pers->grid;
     switch (variant) {
       case kEnsTileRing8:
         k_ens_fluid_tile_persist<TVISCO, TDDT, 8, EOS7><<<g, 64, 0, ctx->stream>>>(
-            cases, st, wmap, nb, pers->chunk, pers->ctr, dcell, poscell, posf, velrho, press,
+            cases, st, wmap, nb, pers->chunk, pers->ctr, dcell, poscell, velrho, press,
             viscdt, ar, ace);
         break;
       case kEnsTileRing12:
         k_ens_fluid_tile_persist<TVISCO, TDDT, 12, EOS7><<<g, 64, 0, ctx->stream>>>(
-            cases, st, wmap, nb, pers->chunk, pers->ctr, dcell, poscell, posf, velrho, press,
+            cases, st, wmap, nb, pers->chunk, pers->ctr, dcell, poscell, velrho, press,
             viscdt, ar, ace);
         break;
       default:
         k_ens_fluid_tile_persist<TVISCO, TDDT, 16, EOS7><<<g, 64, 0, ctx->stream>>>(
-            cases, st, wmap, nb, pers->chunk, pers->ctr, dcell, poscell, posf, velrho, press,
+            cases, st, wmap, nb, pers->chunk, pers->ctr, dcell, poscell, velrho, press,
             viscdt, ar, ace);
         break;
     }
@@ -1834,15 +1861,15 @@ void launch_ens_fluid(dsph_ctx* ctx, int variant, const EnsCase* cases, const En
   switch (variant) {
     case kEnsTileRing8:
       k_ens_fluid_tile<TVISCO, TDDT, 8, EOS7><<<nb, 64, 0, ctx->stream>>>(
-          cases, st, wmap, dcell, poscell, posf, velrho, press, viscdt, ar, ace);
+          cases, st, wmap, dcell, poscell, velrho, press, viscdt, ar, ace);
       break;
     case kEnsTileRing12:
       k_ens_fluid_tile<TVISCO, TDDT, 12, EOS7><<<nb, 64, 0, ctx->stream>>>(
-          cases, st, wmap, dcell, poscell, posf, velrho, press, viscdt, ar, ace);
+          cases, st, wmap, dcell, poscell, velrho, press, viscdt, ar, ace);
       break;
     case kEnsTileRing16:
       k_ens_fluid_tile<TVISCO, TDDT, 16, EOS7><<<nb, 64, 0, ctx->stream>>>(
-          cases, st, wmap, dcell, poscell, posf, velrho, press, viscdt, ar, ace);
+          cases, st, wmap, dcell, poscell, velrho, press, viscdt, ar, ace);
       break;
     default:
       k_ens_fluid_rows<TVISCO, TDDT><<<nb, 64, 0, ctx->stream>>>(
@@ -1856,11 +1883,10 @@ void launch_ens_fluid(dsph_ctx* ctx, int variant, const EnsCase* cases, const En
 namespace dsph {
 
 int ens_prep(dsph_ctx* ctx, const EnsCase* cases, const EnsState* st, const EnsBlock* pmap,
-             unsigned npblocks, const float4* poscell, const float4* velrho, float2* press,
-             float4* posf) {
+             unsigned npblocks, const float4* velrho, float2* press) {
   if (!npblocks) return DSPH_OK;
   KTimer kt(ctx, "k_prep");
-  k_ens_prep<<<npblocks, kBs, 0, ctx->stream>>>(cases, st, pmap, poscell, velrho, press, posf);
+  k_ens_prep<<<npblocks, kBs, 0, ctx->stream>>>(cases, st, pmap, velrho, press);
   DSPH_LAUNCHED(ctx, "k_ens_prep");
   return DSPH_OK;
 }
@@ -1869,7 +1895,7 @@ int ens_forces_fluid(dsph_ctx* ctx, int variant, int tvisco, int tddt, bool eos7
                      const EnsCase* cases, const EnsState* st, const EnsBlock* wmap,
                      unsigned nblocks, const EnsPersist* pers, const unsigned* dcell,
                      const float4* poscell,
-                     const float4* posf, const float4* velrho, const float2* press,
+                     const float4* velrho, const float2* press,
                      float* viscdt, float* ar, float* ace) {
   if (!nblocks) return DSPH_OK;
   DSPH_REQUIRE(ctx, variant >= 0 && variant < kEnsNumVariants, "ensemble: invalid kernel variant");
@@ -1884,9 +1910,9 @@ int ens_forces_fluid(dsph_ctx* ctx, int variant, int tvisco, int tddt, bool eos7
   KTimer kt(ctx, "k_forces_fluid");
 #define DSPH_ENS_FLUID(V, D)                                                              \
   (eos7 ? launch_ens_fluid<V, D, true>(ctx, variant, cases, st, wmap, nblocks, pers, dcell,   \
-                                       poscell, posf, velrho, press, viscdt, ar, ace)         \
+                                       poscell, velrho, press, viscdt, ar, ace)         \
         : launch_ens_fluid<V, D, false>(ctx, variant, cases, st, wmap, nblocks, pers, dcell,  \
-                                        poscell, posf, velrho, press, viscdt, ar, ace))
+                                        poscell, velrho, press, viscdt, ar, ace))
   if (tvisco == DSPH_VISCO_ARTIFICIAL && tddt == DSPH_DDT_DDT2FULL)
     DSPH_ENS_FLUID(DSPH_VISCO_ARTIFICIAL, DSPH_DDT_DDT2FULL);
   else if (tvisco == DSPH_VISCO_ARTIFICIAL && tddt == DSPH_DDT_NONE)
@@ -1931,16 +1957,6 @@ int ens_forces_bound_tile(dsph_ctx* ctx, const EnsCase* cases, const EnsState* s
   k_ens_bound_team<<<nblocks * kTeam, 64, 0, ctx->stream>>>(cases, st, bmap64, A);
   DSPH_LAUNCHED(ctx, "k_ens_bound_team");
   return DSPH_OK;
-}
-
-// Radius^2 of the conservative scan test for a case (see scan_radius2).
-float ens_scan_radius2(const dsph_cte& cte) {
-  const Cte c = make_cte(cte);
-  const double lmax = std::max(std::max(cte.maprealsizex, cte.maprealsizey), cte.maprealsizez) +
-                      2.0 * c.pcs;
-  const double ulp = lmax * 1.1920928955078125e-7;
-  const double r = std::sqrt(double(c.ks2)) + 4.0 * ulp + 1e-6 * std::sqrt(double(c.ks2));
-  return float(r * r);
 }
 
 }  // namespace dsph
@@ -1993,9 +2009,9 @@ int check_inter_parms(dsph_ctx* ctx, const dsph_inter_parms* t) {
   return DSPH_OK;
 }
 
-// The interaction with the per-particle preparation in press/posf (np
-// entries each): k_prep, the fluid kernel, the boundary kernel.
-int interaction_forces(dsph_ctx* ctx, const dsph_inter_parms* t, float2* press, float4* posf) {
+// The interaction with the per-particle preparation in press (np
+// entries): k_prep, the fluid kernel, the boundary kernel.
+int interaction_forces(dsph_ctx* ctx, const dsph_inter_parms* t, float2* press) {
   const Cte c = make_cte(ctx->cte);
   const DivData dvd = make_divdata(t->divdata);
   const unsigned npf = t->np - t->npb;
@@ -2004,22 +2020,21 @@ int interaction_forces(dsph_ctx* ctx, const dsph_inter_parms* t, float2* press, 
     {
       KTimer kt(ctx, "k_prep");
       k_prep<<<grid_for(t->np, kBs), kBs, 0, ctx->stream>>>(
-          t->np, (const float4*)t->d_poscell, (const float4*)t->d_velrho, press,
-          fluid_form(ctx, t) == FluidForm::kTile ? posf : nullptr, c);
+          t->np, (const float4*)t->d_velrho, press, c);
     }
     const bool vg = t->d_velgrad != nullptr;
     switch (t->tvisco) {
       case DSPH_VISCO_ARTIFICIAL:
-        rc = vg ? dispatch_ddt<DSPH_VISCO_ARTIFICIAL, true>(ctx, t, dvd, c, press, posf)
-                : dispatch_ddt<DSPH_VISCO_ARTIFICIAL, false>(ctx, t, dvd, c, press, posf);
+        rc = vg ? dispatch_ddt<DSPH_VISCO_ARTIFICIAL, true>(ctx, t, dvd, c, press)
+                : dispatch_ddt<DSPH_VISCO_ARTIFICIAL, false>(ctx, t, dvd, c, press);
         break;
       case DSPH_VISCO_LAMINAR:
-        rc = vg ? dispatch_ddt<DSPH_VISCO_LAMINAR, true>(ctx, t, dvd, c, press, posf)
-                : dispatch_ddt<DSPH_VISCO_LAMINAR, false>(ctx, t, dvd, c, press, posf);
+        rc = vg ? dispatch_ddt<DSPH_VISCO_LAMINAR, true>(ctx, t, dvd, c, press)
+                : dispatch_ddt<DSPH_VISCO_LAMINAR, false>(ctx, t, dvd, c, press);
         break;
       case DSPH_VISCO_LAMINARSPS:
-        rc = vg ? dispatch_ddt<DSPH_VISCO_LAMINARSPS, true>(ctx, t, dvd, c, press, posf)
-                : dispatch_ddt<DSPH_VISCO_LAMINARSPS, false>(ctx, t, dvd, c, press, posf);
+        rc = vg ? dispatch_ddt<DSPH_VISCO_LAMINARSPS, true>(ctx, t, dvd, c, press)
+                : dispatch_ddt<DSPH_VISCO_LAMINARSPS, false>(ctx, t, dvd, c, press);
         break;
       default: return set_error(ctx, DSPH_E_ARG, "dsph_interaction_forces: invalid tvisco");
     }
@@ -2051,12 +2066,11 @@ int interaction_forces(dsph_ctx* ctx, const dsph_inter_parms* t, float2* press, 
 }
 
 // Scratch of dsph_interaction_forces_noalloc: {press, 1/rho} (float2) for
-// DSPH_NOALLOC_NP_MAX particles, then their map-frame positions (float4).
+// DSPH_NOALLOC_NP_MAX particles.
 // Every GPU holds its own copy for the life of the process; host code uses
 // the device address that hipGetSymbolAddress gives on each device, never
 // the array's name.
-constexpr size_t kNoallocPressBytes = size_t(DSPH_NOALLOC_NP_MAX) * sizeof(float2);
-constexpr size_t kNoallocBytes = kNoallocPressBytes + size_t(DSPH_NOALLOC_NP_MAX) * sizeof(float4);
+constexpr size_t kNoallocBytes = size_t(DSPH_NOALLOC_NP_MAX) * sizeof(float2);
 static __device__ __align__(256) unsigned char scratch[kNoallocBytes];
 
 }  // namespace
@@ -2095,8 +2109,7 @@ int dsph_interaction_forces(dsph_ctx* ctx, const dsph_inter_parms* t) {
     rc = ensure_prep_scratch(ctx, t->np);
     if (rc) return rc;
   }
-  return interaction_forces(ctx, t, reinterpret_cast<float2*>(ctx->prep_press),
-                            reinterpret_cast<float4*>(ctx->prep_posf));
+  return interaction_forces(ctx, t, reinterpret_cast<float2*>(ctx->prep_press));
 }
 
 int dsph_interaction_forces_noalloc(dsph_ctx* ctx, const dsph_inter_parms* t) {
@@ -2110,8 +2123,7 @@ int dsph_interaction_forces_noalloc(dsph_ctx* ctx, const dsph_inter_parms* t) {
   if (!ctx->noalloc_scratch)
     return set_error(ctx, DSPH_E_STATE, "no-alloc scratch address not set up for this device");
   unsigned char* base = static_cast<unsigned char*>(ctx->noalloc_scratch);
-  return interaction_forces(ctx, t, reinterpret_cast<float2*>(base),
-                            reinterpret_cast<float4*>(base + kNoallocPressBytes));
+  return interaction_forces(ctx, t, reinterpret_cast<float2*>(base));
 }
 
 }  // extern "C"

@@ -85,7 +85,7 @@ struct dsph_ens {
   double *movxy = nullptr, *movz = nullptr;
   float *velrho = nullptr, *velrho2 = nullptr, *velrhopre = nullptr, *velrhopre2 = nullptr;
   float *poscell = nullptr, *ace = nullptr, *ar = nullptr, *viscdt = nullptr;
-  float *press = nullptr, *posf = nullptr;
+  float* press = nullptr;
   int* begincell = nullptr;
   bool pre_active = false;
   bool use_graph = true;
@@ -184,7 +184,6 @@ struct dsph_ens {
       e.rhopoutmin = g.RhopOutMin; e.rhopoutmax = g.RhopOutMax;
       e.viscob = g.Visco * g.ViscoBoundFactor;
       e.viscof = g.Visco;
-      e.ks2scan = dsph::ens_scan_radius2(cte);
       e.kernelh = double(g.KernelH);
       e.cs0 = g.Cs0;
       e.cfl = g.CFLnumber;
@@ -235,10 +234,9 @@ struct dsph_ens {
     for (auto& e : hc)
       e.dvd.begincell = reinterpret_cast<const int2*>(begincell) + e.key0;
     // Sort, reduction and interaction scratch of the context ({press, 1/rho}
-    // and map-frame positions per particle).
+    // per particle).
     chk(dsph_ctx_reserve(ctx, ntot, nkeys), "dsph_ctx_reserve");
     press = ctx->prep_press;
-    posf = ctx->prep_posf;
     chk(dsph_memcpy_h2d(ctx, idp, h_idp, 4 * n), "upload idp");
     chk(dsph_memcpy_h2d(ctx, code, hcode.data(), 2 * n), "upload code");
     chk(dsph_memcpy_h2d(ctx, dcell, hdcell.data(), 4 * n), "upload dcell");
@@ -336,8 +334,8 @@ struct dsph_ens {
       chk(dsph::ens_reduce(ctx, d_cases, d_st, d_pmap, npblocks, 0, (const float4*)velrho,
                            viscdt, ace),
           "velmax");
-    chk(dsph::ens_prep(ctx, d_cases, d_st, d_pmap, npblocks, (const float4*)poscell,
-                       (const float4*)velrho, (float2*)press, (float4*)posf),
+    chk(dsph::ens_prep(ctx, d_cases, d_st, d_pmap, npblocks, (const float4*)velrho,
+                       (float2*)press),
         "prep");
   }
 
@@ -352,8 +350,8 @@ struct dsph_ens {
     }
     chk(dsph::ens_forces_fluid(ctx, variant, tvisco, tddt, eos7, d_cases, d_st, bk.d_wmap,
                                bk.nblocks, chunk ? &pers : nullptr,
-                               dcell, (const float4*)poscell, (const float4*)posf,
-                               (const float4*)velrho, (const float2*)press, viscdt, ar, ace),
+                               dcell, (const float4*)poscell, (const float4*)velrho,
+                               (const float2*)press, viscdt, ar, ace),
         "fluid interaction");
   }
   void fluid_tuned(unsigned b) {
