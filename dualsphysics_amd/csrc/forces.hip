@@ -1555,14 +1555,13 @@ enum class FluidForm { kTeam, kTile, kRows };
 
 // Form of the fluid interaction (all give the same bits).
 // Teams win while the chip is not full of the tile kernel's waves of 64
-// particles, the tile kernel (fewer instructions per pair, 5 waves per SIMD
-// against 3) above. Measured, us, team / tile:
-//   artificial  3-D   10k fluid particles 115 / 467,  80k 251 / 511, 234k 573 / 645,
-//                     643k 1392 / 1198
-//   laminar     3-D   80k 275 / 506, 234k 645 / 656, 643k 1575 / 1202
-//   Laminar+SPS 3-D   80k 455 / 616, 157k 781 / 685
-//   artificial  2-D (step)  120k 473 / 498, 480k 769 / 699
-//   mDBC2 (laminar, step)   122k 2036 / 2375, 372k 3927 / 3894
+// particles, the tile kernel (5 waves per SIMD against 3, fewer LDS accesses
+// per pair) above. Measured, us, team / tile:
+//   artificial  3-D   80k fluid particles 253 / 379, 157k 424 / 443, 234k 591 / 528
+//   laminar     3-D   80k 280 / 378, 157k 467 / 437, 234k 656 / 519
+//   Laminar+SPS 3-D   80k 451 / 490, 157k 781 / 565
+//   artificial  2-D (step)  120k 453 / 465, 480k 769 / 662
+//   mDBC2 (laminar, step)   122k 1466 / 1567
 // Floating bodies have no tile kernel; against rows: 92k 1020 / 2286 (step),
 // 380k 2640 / 3343. Shifting has no team kernel: which boundary neighbour
 // cancels it first decides what is summed.
@@ -1571,11 +1570,11 @@ FluidForm fluid_form(const dsph_ctx* ctx, const dsph_inter_parms* t) {
   if (t->d_ftomassp) return FluidForm::kTeam;
   if (t->d_boundmode && (t->d_shiftposfs || t->d_velgrad)) return FluidForm::kRows;
   if (t->d_shiftposfs || t->d_velgrad) return FluidForm::kTile;
-  const unsigned most = t->tvisco == DSPH_VISCO_ARTIFICIAL ? 320000u
-                        : t->tvisco == DSPH_VISCO_LAMINAR  ? 240000u
-                                                           : 120000u;
+  const unsigned most = t->tvisco == DSPH_VISCO_ARTIFICIAL ? 180000u
+                        : t->tvisco == DSPH_VISCO_LAMINAR  ? 140000u
+                                                           : 100000u;
   const unsigned npf = t->np - t->npb;
-  return npf <= (ctx->cte.simulate2d ? most / 2 : most) ? FluidForm::kTeam : FluidForm::kTile;
+  return npf <= (ctx->cte.simulate2d ? most / 4 * 3 : most) ? FluidForm::kTeam : FluidForm::kTile;
 }
 
 template <int TVISCO, int TDDT, bool VELGRAD>
