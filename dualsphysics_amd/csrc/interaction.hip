@@ -9,7 +9,6 @@ using namespace dsph;
 
 namespace {
 
-constexpr unsigned kBsForces = 128;
 constexpr unsigned kBs = 256;
 
 // Smagorinsky + Blin SPS stress tau/rho^2 (KerComputeSpsTau, JSphGpu_ker.cu:1387-1420).
@@ -119,65 +118,184 @@ __device__ inline double mdbc_det_inv(bool sim2d, const M4d& a, M4d& inv) {
   return det;
 }
 
+// ------------------------------------------------------------ sums at the ghost nodes
+// 16 lanes work on one ghost node: they test 16 neighbours of a row at a time,
+// each evaluates the terms of its hit and appends their factors, in row
+// order, to LDS, and every lane then adds its own component of the sums over the hits
+// one after the other (lane 4 i + j: A[i][j]; the first lanes the others too). Each
+// sum runs in the order of one lane walking the rows, with its roundings:
+// identical bits. One lane per ghost node was a serial chain of some 700
+// gathers on few waves. mDBC2 step of 200k particles 2.04 -> 1.50 ms (78k
+// boundary particles: 428 us a call before); where many walls fill the chip
+// (wave flume, 0.6M boundary particles) 567 -> 518 us, bound by the VALU.
+constexpr unsigned kGhostLanes = 16, kGhosts = 16;   // lanes per ghost, ghosts per workgroup
+constexpr unsigned kGhostBs = kGhostLanes * kGhosts;
+constexpr unsigned kGhostRec = 20;   // floats per record: F[4], D[4], Q[8], {-volume}
+constexpr unsigned kGhostUnroll = 4;
+
+struct GhostSums {
+  float A[4][4];                // kernel and its gradient times {1, dr} (mDBC2: -dr)
+  float rhop, grx, gry, grz;    // sum m W, sum m gradW
+  float vpx, vpy, vpz;          // mDBC2: sum V W v
+  float submerged;              // mDBC2: -sum V dr.gradW
+};
+static_assert(sizeof(GhostSums) == 24 * sizeof(float), "written lane by lane");
+
+struct GhostLds {
+  float rec[kGhostBs * kGhostRec];
+  GhostSums sums[kGhosts];
+};
+
+__device__ __forceinline__ void ghost_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Sums of the ghost node of boundary particle p1 (without one unless active),
+// left in lds.sums[threadIdx.x / 16] for the caller behind a barrier.
+template <bool MDBC2>
+__device__ __forceinline__ void ghost_sums(bool active, unsigned p1, float bnx, float bny,
+    float bnz, const DivData& dvd, const Cte& c, const double3& mapposmin,
+    const double2* __restrict__ posxy, const double* __restrict__ posz,
+    const float4* __restrict__ poscell, const typecode* __restrict__ code,
+    const float4* __restrict__ velrho, GhostLds& lds) {
+  const unsigned lane = threadIdx.x & 63u, r = lane & (kGhostLanes - 1), g = lane / kGhostLanes;
+  float* const rec = lds.rec + (threadIdx.x / kGhostLanes) * kGhostLanes * kGhostRec;
+  float4 gps = make_float4(0, 0, 0, 0);
+  NgLimits l = {0, 0, 0, 0, 0, 0};
+  if (active) {
+    // PosCell of the ghost node (KerComputePosCell, JSphGpu_ker.cu:1185-1202)
+    // and its cell: an FP64 quotient each for x, y, z, on lanes 0..2 and 4..6.
+    const unsigned ax = r & 3u;
+    const double gp = ax == 0 ? posxy[p1].x + bnx : (ax == 1 ? posxy[p1].y + bny : posz[p1] + bnz);
+    const double mapmin = ax == 0 ? mapposmin.x : (ax == 1 ? mapposmin.y : mapposmin.z);
+    const double dommin = ax == 0 ? dvd.domposminx : (ax == 1 ? dvd.domposminy : dvd.domposminz);
+    const bool map = r < 4;
+    const double num = gp - (map ? mapmin : dommin);
+    const double quo = num / (map ? double(c.pcs) : double(dvd.scell));
+    const int cell = map ? int(unsigned(quo)) : int(quo);
+    const float rest = float(num - double(c.pcs) * unsigned(cell));
+    const int l0 = int(g * kGhostLanes);
+    gps = make_float4(__shfl(rest, l0), __shfl(rest, l0 + 1), __shfl(rest, l0 + 2),
+                      __uint_as_float(pscel_code(unsigned(__shfl(cell, l0)),
+                                                 unsigned(__shfl(cell, l0 + 1)),
+                                                 unsigned(__shfl(cell, l0 + 2)))));
+    l = ng_limits(__shfl(cell, l0 + 4) - dvd.czx, __shfl(cell, l0 + 5) - dvd.czy,
+                  __shfl(cell, l0 + 6) - dvd.czz, dvd);
+  }
+  const int ny = max(l.y1 - l.y0, 0), nrows = ny * max(l.z1 - l.z0, 0);
+  // This lane's sums: A[r / 4][r % 4], and for r < 8 member r of the others.
+  float a = 0.f, b = 0.f;
+  const unsigned fi = r >> 2, dj = 4 + (r & 3u), qr = 8 + (r & 7u);
+  int row = 0;                       // next row of the node
+  unsigned rini = 0, rfin = 0;       // rows row - row % 16 + lane
+  unsigned t = 0, tfin = 0;
+  for (;;) {
+    // Next row that is not empty (the same on the node's lanes).
+    bool more = t < tfin;
+    while (__ballot(!more && row < nrows)) {
+      if ((row & 15) == 0 && !more && row < nrows) {
+        const int ri = row + int(r);
+        rini = rfin = 0;
+        if (ri < nrows) {
+          const int z = l.z0 + ri / ny, y = l.y0 + ri % ny;
+          row_range(dvd.begincell, int(dvd.cellfluid) + z * dvd.ncw + y * dvd.ncx, l.x0, l.x1,
+                    rini, rfin);
+        }
+      }
+      const int src = int(g * kGhostLanes) + (row & 15);
+      const unsigned t0 = unsigned(__shfl(int(rini), src)), t1 = unsigned(__shfl(int(rfin), src));
+      if (!more && row < nrows) {
+        t = t0;
+        tfin = t1;
+        row++;
+        more = t < tfin;
+      }
+    }
+    if (!__ballot(more)) break;
+    const bool in = more && t + r < tfin;
+    const unsigned p2 = in ? t + r : 0u;
+    t += kGhostLanes;
+    bool hit = false;
+    float3 dr = make_float3(0, 0, 0);
+    float rr2 = 0.f;
+    if (in) {
+      dr = pscel_dr(gps, poscell[p2], c.pcs);
+      rr2 = dr.x * dr.x + dr.y * dr.y + dr.z * dr.z;
+      hit = rr2 <= c.ks2 && code_is_fluid(code[p2]);
+    }
+    const unsigned hits = unsigned(__ballot(hit) >> (g * kGhostLanes)) & 0xffffu;
+    const unsigned nhit = unsigned(__popc(hits));
+    ghost_sync();
+    if (hit) {
+      float fac;
+      const float wab = wendland_wab_fac(rr2, c, fac);
+      const float frx = fac * dr.x, fry = fac * dr.y, frz = fac * dr.z;
+      const float4 vr2 = velrho[p2];
+      const float volp2 = c.massf / vr2.w;
+      float4* const o = reinterpret_cast<float4*>(
+          rec + unsigned(__popc(hits & ((1u << r) - 1u))) * kGhostRec);
+      o[0] = make_float4(wab * volp2, frx * volp2, fry * volp2, frz * volp2);
+      o[1] = MDBC2 ? make_float4(1.f, -dr.x, -dr.y, -dr.z) : make_float4(1.f, dr.x, dr.y, dr.z);
+      o[2] = make_float4(wab, frx, fry, frz);
+      if (MDBC2) {
+        o[3] = make_float4(vr2.x, vr2.y, vr2.z, dr.x * frx + dr.y * fry + dr.z * frz);
+        o[4].x = -volp2;
+      }
+    }
+    ghost_sync();
+    for (unsigned k = 0; __ballot(k < nhit); k += kGhostUnroll) {
+      float F[kGhostUnroll], D[kGhostUnroll], P[kGhostUnroll], Q[kGhostUnroll];
+#pragma unroll
+      for (unsigned u = 0; u < kGhostUnroll; u++) {
+        const float* const q = rec + min(k + u, kGhostLanes - 1) * kGhostRec;
+        F[u] = q[fi];
+        D[u] = q[dj];
+        Q[u] = q[MDBC2 ? qr : 8 + (r & 3u)];
+        P[u] = MDBC2 && r >= 4 ? q[r == 7 ? 16 : 0] : c.massf;
+      }
+#pragma unroll
+      for (unsigned u = 0; u < kGhostUnroll; u++) {
+        const bool is = k + u < nhit;
+        const float an = D[u] * F[u] + a, bn = P[u] * Q[u] + b;
+        a = is ? an : a;
+        b = is ? bn : b;
+      }
+    }
+  }
+  float* const o = reinterpret_cast<float*>(lds.sums + threadIdx.x / kGhostLanes);
+  o[r] = a;
+  if (r < 8) o[16 + r] = b;
+}
+
 // mDBC, SlipMode SLIP_Vel0 (KerInteractionMdbcCorrection_Fast,
 // JSphGpu_mdbc_iker.cu:34-150): Shepard density and gradient at the ghost node
 // g = x_b + boundnor with a first-order (4x4) correction; mirrored back to
 // the boundary particle by a linear extrapolation.
-__global__ void __launch_bounds__(kBsForces) k_mdbc(unsigned n, DivData dvd, Cte c,
+__global__ void __launch_bounds__(kGhostBs) k_mdbc(unsigned n, DivData dvd, Cte c,
     double3 mapposmin, const double2* __restrict__ posxy, const double* __restrict__ posz,
     const float4* __restrict__ poscell, const typecode* __restrict__ code,
     const float* __restrict__ boundnor, float4* __restrict__ velrho) {
-  const unsigned p1 = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p1 >= n) return;
-  const float bnx = boundnor[3 * size_t(p1)], bny = boundnor[3 * size_t(p1) + 1],
-              bnz = boundnor[3 * size_t(p1) + 2];
-  if (bnx == 0 && bny == 0 && bnz == 0) return;
-  const double gx = posxy[p1].x + bnx, gy = posxy[p1].y + bny, gz = posz[p1] + bnz;
-  // PosCell of the ghost node (KerComputePosCell, JSphGpu_ker.cu:1185-1202).
-  float4 gps;
-  {
-    const double dx = gx - mapposmin.x, dy = gy - mapposmin.y, dz = gz - mapposmin.z;
-    const unsigned cx = unsigned(dx / c.pcs), cy = unsigned(dy / c.pcs), cz = unsigned(dz / c.pcs);
-    gps = make_float4(float(dx - double(c.pcs) * cx), float(dy - double(c.pcs) * cy),
-                      float(dz - double(c.pcs) * cz), __uint_as_float(pscel_code(cx, cy, cz)));
-  }
-  float rhop1 = 0, grx = 0, gry = 0, grz = 0;
-  float A[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; i++)
-#pragma unroll
-    for (int j = 0; j < 4; j++) A[i][j] = 0;
-  const int cx = int((gx - dvd.domposminx) / dvd.scell) - dvd.czx;
-  const int cy = int((gy - dvd.domposminy) / dvd.scell) - dvd.czy;
-  const int cz = int((gz - dvd.domposminz) / dvd.scell) - dvd.czz;
-  const NgLimits l = ng_limits(cx, cy, cz, dvd);
-  for (int z = l.z0; z < l.z1; z++)
-    for (int y = l.y0; y < l.y1; y++) {
-      unsigned pini, pfin;
-      row_range(dvd.begincell, int(dvd.cellfluid) + z * dvd.ncw + y * dvd.ncx, l.x0, l.x1,
-                pini, pfin);
-      for (unsigned p2 = pini; p2 < pfin; p2++) {
-        const float4 ps2 = poscell[p2];
-        const float3 dr = pscel_dr(gps, ps2, c.pcs);
-        const float rr2 = dr.x * dr.x + dr.y * dr.y + dr.z * dr.z;
-        if (rr2 <= c.ks2 && code_is_fluid(code[p2])) {
-          float fac;
-          const float wab = wendland_wab_fac(rr2, c, fac);
-          const float frx = fac * dr.x, fry = fac * dr.y, frz = fac * dr.z;
-          const float4 vr2 = velrho[p2];
-          const float massp2 = c.massf;
-          const float volp2 = massp2 / vr2.w;
-          rhop1 += massp2 * wab;
-          grx += massp2 * frx; gry += massp2 * fry; grz += massp2 * frz;
-          const float vwab = wab * volp2, vfrx = frx * volp2, vfry = fry * volp2,
-                      vfrz = frz * volp2;
-          A[0][0] += vwab; A[0][1] += dr.x * vwab; A[0][2] += dr.y * vwab; A[0][3] += dr.z * vwab;
-          A[1][0] += vfrx; A[1][1] += dr.x * vfrx; A[1][2] += dr.y * vfrx; A[1][3] += dr.z * vfrx;
-          A[2][0] += vfry; A[2][1] += dr.x * vfry; A[2][2] += dr.y * vfry; A[2][3] += dr.z * vfry;
-          A[3][0] += vfrz; A[3][1] += dr.x * vfrz; A[3][2] += dr.y * vfrz; A[3][3] += dr.z * vfrz;
-        }
-      }
-    }
+  __shared__ GhostLds lds;
+  auto normal = [&](unsigned p, float& x, float& y, float& z) {
+    if (p >= n) return false;
+    x = boundnor[3 * size_t(p)]; y = boundnor[3 * size_t(p) + 1]; z = boundnor[3 * size_t(p) + 2];
+    return !(x == 0 && y == 0 && z == 0);
+  };
+  float bnx = 0, bny = 0, bnz = 0;
+  const unsigned pl = blockIdx.x * kGhosts + threadIdx.x / kGhostLanes;
+  const bool active = normal(pl, bnx, bny, bnz);
+  ghost_sums<false>(active, pl, bnx, bny, bnz, dvd, c, mapposmin, posxy, posz, poscell, code,
+                    velrho, lds);
+  __syncthreads();
+  // One lane per node from here on.
+  if (threadIdx.x >= kGhosts) return;
+  const unsigned p1 = blockIdx.x * kGhosts + threadIdx.x;
+  if (!normal(p1, bnx, bny, bnz)) return;
+  const GhostSums S = lds.sums[threadIdx.x];
+  const auto& A = S.A;
+  const float rhop1 = S.rhop, grx = S.grx, gry = S.gry, grz = S.grz;
   float rhofinal = FLT_MAX;
   M4d Ad, inv;
 #pragma unroll
@@ -221,71 +339,38 @@ __device__ inline float3 mdbc2_tangential(float bx, float by, float bz, float3 v
   return make_float3(v.x - vdn * nx, v.y - vdn * ny, v.z - vdn * nz);
 }
 
-__global__ void __launch_bounds__(kBsForces) k_mdbc2(unsigned n, int tslip, DivData dvd, Cte c,
+__global__ void __launch_bounds__(kGhostBs) k_mdbc2(unsigned n, int tslip, DivData dvd, Cte c,
     float3 gravity, double3 mapposmin, const double2* __restrict__ posxy,
     const double* __restrict__ posz, const float4* __restrict__ poscell,
     const typecode* __restrict__ code, const float* __restrict__ boundnor,
     const float* __restrict__ motionvel, const float* __restrict__ motionace,
     float4* __restrict__ velrho, uint8_t* __restrict__ boundmode, float* __restrict__ tangenvel) {
-  const unsigned p1 = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p1 >= n) return;
-  const float bnx = boundnor[3 * size_t(p1)], bny = boundnor[3 * size_t(p1) + 1],
-              bnz = boundnor[3 * size_t(p1) + 2];
-  if (bnx == 0 && bny == 0 && bnz == 0) return;
+  __shared__ GhostLds lds;
+  auto normal = [&](unsigned p, float& x, float& y, float& z) {
+    if (p >= n) return false;
+    x = boundnor[3 * size_t(p)]; y = boundnor[3 * size_t(p) + 1]; z = boundnor[3 * size_t(p) + 2];
+    return !(x == 0 && y == 0 && z == 0);
+  };
+  float bnx = 0, bny = 0, bnz = 0;
+  const unsigned pl = blockIdx.x * kGhosts + threadIdx.x / kGhostLanes;
+  const bool active = normal(pl, bnx, bny, bnz);
+  ghost_sums<true>(active, pl, bnx, bny, bnz, dvd, c, mapposmin, posxy, posz, poscell, code,
+                   velrho, lds);
+  __syncthreads();
+  // One lane per node from here on.
+  if (threadIdx.x >= kGhosts) return;
+  const unsigned p1 = blockIdx.x * kGhosts + threadIdx.x;
+  if (!normal(p1, bnx, bny, bnz)) return;
+  const GhostSums S = lds.sums[threadIdx.x];
+  const auto& A = S.A;
+  const float rhop1 = S.rhop, grx = S.grx, gry = S.gry, grz = S.grz, sumwab = A[0][0],
+              submerged = S.submerged, vpx = S.vpx, vpy = S.vpy, vpz = S.vpz;
   const float3 mv = motionvel ? make_float3(motionvel[3 * size_t(p1)], motionvel[3 * size_t(p1) + 1],
                                             motionvel[3 * size_t(p1) + 2])
                               : make_float3(0, 0, 0);
   const float3 ma = motionace ? make_float3(motionace[3 * size_t(p1)], motionace[3 * size_t(p1) + 1],
                                             motionace[3 * size_t(p1) + 2])
                               : make_float3(0, 0, 0);
-  const double gx = posxy[p1].x + bnx, gy = posxy[p1].y + bny, gz = posz[p1] + bnz;
-  float4 gps;
-  {
-    const double dx = gx - mapposmin.x, dy = gy - mapposmin.y, dz = gz - mapposmin.z;
-    const unsigned cx = unsigned(dx / c.pcs), cy = unsigned(dy / c.pcs), cz = unsigned(dz / c.pcs);
-    gps = make_float4(float(dx - double(c.pcs) * cx), float(dy - double(c.pcs) * cy),
-                      float(dz - double(c.pcs) * cz), __uint_as_float(pscel_code(cx, cy, cz)));
-  }
-  float rhop1 = 0, grx = 0, gry = 0, grz = 0, sumwab = 0, submerged = 0;
-  float vpx = 0, vpy = 0, vpz = 0;
-  float A[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; i++)
-#pragma unroll
-    for (int j = 0; j < 4; j++) A[i][j] = 0;
-  const int cx = int((gx - dvd.domposminx) / dvd.scell) - dvd.czx;
-  const int cy = int((gy - dvd.domposminy) / dvd.scell) - dvd.czy;
-  const int cz = int((gz - dvd.domposminz) / dvd.scell) - dvd.czz;
-  const NgLimits l = ng_limits(cx, cy, cz, dvd);
-  for (int z = l.z0; z < l.z1; z++)
-    for (int y = l.y0; y < l.y1; y++) {
-      unsigned pini, pfin;
-      row_range(dvd.begincell, int(dvd.cellfluid) + z * dvd.ncw + y * dvd.ncx, l.x0, l.x1,
-                pini, pfin);
-      for (unsigned p2 = pini; p2 < pfin; p2++) {
-        const float4 ps2 = poscell[p2];
-        const float3 dr = pscel_dr(gps, ps2, c.pcs);
-        const float rr2 = dr.x * dr.x + dr.y * dr.y + dr.z * dr.z;
-        if (rr2 <= c.ks2 && code_is_fluid(code[p2])) {
-          float fac;
-          const float wab = wendland_wab_fac(rr2, c, fac);
-          const float frx = fac * dr.x, fry = fac * dr.y, frz = fac * dr.z;
-          const float4 vr2 = velrho[p2];
-          const float volp2 = c.massf / vr2.w;
-          submerged -= volp2 * (dr.x * frx + dr.y * fry + dr.z * frz);
-          rhop1 += c.massf * wab;
-          grx += c.massf * frx; gry += c.massf * fry; grz += c.massf * frz;
-          const float vwab = wab * volp2;
-          sumwab += vwab;
-          const float vfrx = frx * volp2, vfry = fry * volp2, vfrz = frz * volp2;
-          vpx += vwab * vr2.x; vpy += vwab * vr2.y; vpz += vwab * vr2.z;
-          A[0][0] += vwab; A[0][1] -= dr.x * vwab; A[0][2] -= dr.y * vwab; A[0][3] -= dr.z * vwab;
-          A[1][0] += vfrx; A[1][1] -= dr.x * vfrx; A[1][2] -= dr.y * vfrx; A[1][3] -= dr.z * vfrx;
-          A[2][0] += vfry; A[2][1] -= dr.x * vfry; A[2][2] -= dr.y * vfry; A[2][3] -= dr.z * vfry;
-          A[3][0] += vfrz; A[3][1] -= dr.x * vfrz; A[3][2] -= dr.y * vfrz; A[3][3] -= dr.z * vfrz;
-        }
-      }
-    }
   float* tv = tangenvel + 3 * size_t(p1);
   if (!(submerged > 0.f)) {
     boundmode[p1] = DSPH_BMODE_MDBC2OFF;
@@ -576,7 +661,7 @@ int dsph_mdbc_correction(dsph_ctx* ctx, uint32_t n, const dsph_divdata* dvdp,
   DSPH_REQUIRE(ctx, d_posxy && d_posz && d_poscell && d_code && d_boundnor && d_velrho,
                "dsph_mdbc_correction: null array");
   const Cte c = make_cte(ctx->cte);
-  k_mdbc<<<grid_for(n, kBsForces), kBsForces, 0, ctx->stream>>>(
+  k_mdbc<<<grid_for(n, kGhosts), kGhostBs, 0, ctx->stream>>>(
       n, make_divdata(*dvdp), c, make_double3(mapposmin[0], mapposmin[1], mapposmin[2]),
       (const double2*)d_posxy, d_posz, (const float4*)d_poscell, d_code, d_boundnor,
       (float4*)d_velrho);
@@ -611,7 +696,7 @@ int dsph_mdbc2_correction_slip(dsph_ctx* ctx, int32_t slipmode, uint32_t n,
                         d_boundmode && d_tangenvel,
                "dsph_mdbc2_correction: null array");
   const Cte c = make_cte(ctx->cte);
-  k_mdbc2<<<grid_for(n, kBsForces), kBsForces, 0, ctx->stream>>>(
+  k_mdbc2<<<grid_for(n, kGhosts), kGhostBs, 0, ctx->stream>>>(
       n, slipmode, make_divdata(*dvdp), c, make_float3(gravity[0], gravity[1], gravity[2]),
       make_double3(mapposmin[0], mapposmin[1], mapposmin[2]), (const double2*)d_posxy, d_posz,
       (const float4*)d_poscell, d_code, d_boundnor, d_motionvel, d_motionace, (float4*)d_velrho,

@@ -85,3 +85,15 @@ def test_mdbc_correction_matches_oracle(lib, ctx, name):
                  (pb[:, 0] < 0.45) & (pb[:, 1] > 0.15) & (pb[:, 1] < 0.45))
         rho_exact = c.rhop0 + c.rhop0 * 9.81 * (DEPTH - pb[:, 2]) / c.cs0 ** 2
         assert np.abs(g[:npb, 3] - rho_exact)[inner].max() < TOL_RHO
+
+
+@pytest.mark.parametrize("m", [1, 15, 16, 17, 67])
+def test_mdbc_correction_of_a_part(lib, ctx, m):
+    """The first m boundary particles alone (16 ghost nodes a workgroup): the
+    same bits as with all of them, the others untouched."""
+    p = casemod.Parameters(tboundary=N.BC_MDBC, tvisco=N.VISCO_LAMINARSPS, visco=1e-6)
+    s = mdbc2_state(perturbed_case(casemod.dam_break(dp=0.02, params=p)))
+    full, part = _gpu_mdbc(lib, ctx, s), _gpu_mdbc(lib, ctx, dict(s, npb=m))
+    assert np.any(full[:17, 3] != s["d"]["velrho"][:17, 3])
+    np.testing.assert_array_equal(part[:m].view(np.uint32), full[:m].view(np.uint32))
+    np.testing.assert_array_equal(part[m:], s["d"]["velrho"][m:])
