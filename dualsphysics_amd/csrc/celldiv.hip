@@ -165,18 +165,25 @@ __global__ void __launch_bounds__(kBs) k_presort_fluid(unsigned n, unsigned pini
 // ballot per digit bit, and keeps per-wave digit counters in LDS. A per-digit
 // scan over waves and over tiles (digit-major histogram) gives each key its
 // global slot.
-constexpr unsigned kTileItems = 16;
-constexpr unsigned kTile = kBs * kTileItems;  // 4096
+// Keys per lane of a tile. Ranking is a serial chain of kItems rounds through the
+// digit counters, so up to 2^21 keys
+// take short tiles, which also put more workgroups on the chip. Scatter, 16 -> 4
+// keys per lane: 1.7k keys 13 -> 6.0 us, 141k 18.3 -> 7.3, 1.1M 22.4 -> 12.7; whole
+// pass of 3.0M keys 38.3 -> 39.4 us (more histogram entries to scan).
+constexpr unsigned kItemsLong = 16, kItemsShort = kSortShortTile / kBs;
+static_assert(kBs * kItemsLong == kSortTile, "sort_scratch_words counts these tiles");
 
+template <unsigned kItems>
 __global__ void __launch_bounds__(kBs) k_radix_hist(const unsigned* __restrict__ keys,
     unsigned n, unsigned shift, unsigned mask, unsigned ntiles, unsigned* __restrict__ hist) {
+  constexpr unsigned kTile = kBs * kItems;
   __shared__ unsigned cnt[256];
   const unsigned tile = blockIdx.x;
   cnt[threadIdx.x] = 0;
   __syncthreads();
   const unsigned base = tile * kTile;
 #pragma unroll
-  for (unsigned i = 0; i < kTileItems; i++) {
+  for (unsigned i = 0; i < kItems; i++) {
     const unsigned idx = base + i * kBs + threadIdx.x;
     if (idx < n) atomicAdd(&cnt[(keys[idx] >> shift) & mask], 1u);
   }
@@ -221,10 +228,12 @@ __global__ void __launch_bounds__(kBs) k_radix_scan_digit(unsigned* __restrict__
 // then writes every digit run with consecutive threads on consecutive
 // addresses: one coalesced store per run instead of one store per key at its
 // own global slot.
+template <unsigned kItems>
 __global__ void __launch_bounds__(kBs) k_radix_scatter(const unsigned* __restrict__ kin,
     const unsigned* __restrict__ vin, unsigned* __restrict__ kout, unsigned* __restrict__ vout,
     unsigned n, unsigned shift, unsigned bits, unsigned ntiles,
     const unsigned* __restrict__ hist, const unsigned* __restrict__ totals) {
+  constexpr unsigned kTile = kBs * kItems;
   __shared__ unsigned dbase[256];           // global slot of the tile's first key of digit d
   __shared__ unsigned lstart[256];          // tile-local position of the first key of digit d
   __shared__ unsigned wcnt[kBs / 64][256];  // per-wave digit counters, then wave offsets
@@ -255,10 +264,10 @@ __global__ void __launch_bounds__(kBs) k_radix_scatter(const unsigned* __restric
   __syncthreads();
   volatile unsigned* cnt = wcnt[w];
   const unsigned seg = w * (kTile / (kBs / 64));   // wave segment, tile-local
-  unsigned key[kTileItems], val[kTileItems], rank[kTileItems];
+  unsigned key[kItems], val[kItems], rank[kItems];
   const unsigned long long lanelt = (1ull << lane) - 1ull;
 #pragma unroll
-  for (unsigned r = 0; r < kTileItems; r++) {
+  for (unsigned r = 0; r < kItems; r++) {
     const unsigned li = seg + r * 64 + lane;
     const bool valid = li < tcount;
     unsigned k = 0, v = 0;
@@ -309,7 +318,7 @@ __global__ void __launch_bounds__(kBs) k_radix_scatter(const unsigned* __restric
   }
   __syncthreads();
 #pragma unroll
-  for (unsigned r = 0; r < kTileItems; r++) {
+  for (unsigned r = 0; r < kItems; r++) {
     if (rank[r] != 0xffffffffu) {
       const unsigned d = (key[r] >> shift) & mask;
       const unsigned lp = lstart[d] + wcnt[w][d] + rank[r];
@@ -658,7 +667,8 @@ int radix_sort(dsph_ctx* ctx, uint32_t* d_keys, uint32_t* d_values, uint32_t n,
   if (bits_total == 0) return DSPH_OK;  // all keys equal (key_limit<=1)
   unsigned *ka_alt = buf, *va_alt = buf + cap, *kb_alt = buf + 2 * cap, *vb_alt = buf + 3 * cap;
   unsigned* hist = buf + 4 * cap;
-  const unsigned ntiles = (n + kTile - 1) / kTile;
+  const bool is_short = n <= kSortShortKeys;
+  const unsigned ntiles = grid_for(n, is_short ? kSortShortTile : kSortTile);
   unsigned* totals = hist + size_t(256) * ntiles;
   unsigned npass = (bits_total + 7) / 8;
   // (shift, bits) of every pass.
@@ -683,10 +693,12 @@ int radix_sort(dsph_ctx* ctx, uint32_t* d_keys, uint32_t* d_values, uint32_t n,
   }
   for (unsigned p = 0; p < npass; p++) {
     const unsigned mask = (1u << bw[p]) - 1u;
-    k_radix_hist<<<ntiles, kBs, 0, ctx->stream>>>(kbuf[p], n, sh[p], mask, ntiles, hist);
+    const auto hist_kernel = is_short ? k_radix_hist<kItemsShort> : k_radix_hist<kItemsLong>;
+    hist_kernel<<<ntiles, kBs, 0, ctx->stream>>>(kbuf[p], n, sh[p], mask, ntiles, hist);
     k_radix_scan_digit<<<mask + 1, kBs, 0, ctx->stream>>>(hist, ntiles, totals);
-    k_radix_scatter<<<ntiles, kBs, 0, ctx->stream>>>(kbuf[p], vbuf[p], kbuf[p + 1], vbuf[p + 1],
-                                                     n, sh[p], bw[p], ntiles, hist, totals);
+    const auto scatter = is_short ? k_radix_scatter<kItemsShort> : k_radix_scatter<kItemsLong>;
+    scatter<<<ntiles, kBs, 0, ctx->stream>>>(kbuf[p], vbuf[p], kbuf[p + 1], vbuf[p + 1], n, sh[p],
+                                             bw[p], ntiles, hist, totals);
     DSPH_LAUNCHED(ctx, "radix pass");
   }
   return DSPH_OK;

@@ -102,10 +102,14 @@ struct KTimer {
 };
 
 // Words of radix-sort scratch for up to cap keys: alternate buffers A and B
-// (keys, values: 4 cap words) and the digit histograms of 4096-key tiles
+// (keys, values: 4 cap words) and the digit histograms of the tiles
 // (256 per tile, plus the digit totals).
+constexpr unsigned kSortTile = 4096, kSortShortTile = 1024;
+constexpr unsigned kSortShortKeys = 1u << 21;   // up to so many keys: short tiles
 constexpr size_t sort_scratch_words(size_t cap) {
-  return 4 * cap + 256 * ((cap + 4095) / 4096 + 1) + 512;
+  const size_t few = cap < kSortShortKeys ? cap : kSortShortKeys;
+  const size_t t = (cap + kSortTile - 1) / kSortTile, ts = (few + kSortShortTile - 1) / kSortShortTile;
+  return 4 * cap + 256 * ((t > ts ? t : ts) + 1) + 512;
 }
 // Ensures ctx scratch can hold a sort of n keys with key_limit.
 int ensure_sort_scratch(dsph_ctx* ctx, uint32_t n);

@@ -31,6 +31,17 @@ def test_sort_random_keys_is_stable(lib, ctx, n, limit):
     np.testing.assert_array_equal(ks, keys[perm])
 
 
+@pytest.mark.parametrize("n", [1023, 1025, 2047, 1 << 21, (1 << 21) + 1])
+def test_sort_tile_edges(lib, ctx, n):
+    """Around one short tile (1024 keys) and around the change to long ones."""
+    assert lib.dsph_ctx_reserve(ctx, n, 1 << 20) == 0
+    keys = np.random.default_rng(n).integers(0, 70000, n).astype(np.uint32)
+    ks, vs = _sort_gpu(lib, ctx, keys, 70000)
+    perm = np.argsort(keys, kind="stable")
+    np.testing.assert_array_equal(vs, perm)
+    np.testing.assert_array_equal(ks, keys[perm])
+
+
 @pytest.mark.parametrize("pattern", ["equal", "sorted", "reversed", "nearly_sorted", "max_key"])
 def test_sort_patterns(lib, ctx, pattern):
     n, limit = 300001, 1 << 20
