@@ -69,7 +69,7 @@ __device__ inline bf16x4 pack4(float a, float b, float c, float d) {
 }
 __device__ inline bf16x4 load_bf4(const unsigned short* p) {
   bf16x4 r;
-  r[0] = (short)p[0]; r[1] = (short)p[1]; r[2] = (short)p[2]; r[3] = (short)p[3];
+  __builtin_memcpy(&r, p, sizeof(r));   // one load, whatever the alignment
   return r;
 }
 // Sum over the 16 lanes of a lane group (same g).
@@ -190,13 +190,12 @@ __device__ inline void load_weights(const unsigned short* __restrict__ wbf,
 #pragma unroll
     for (int kb = 0; kb < 4; kb++)
       w.w2[jb][kb] = load_bf4(wbf + kBfW2 + (jb * 16 + c) * kHid + kb * 16 + 4 * g);
+    const int u = jb * 16 + 4 * g;
+    __builtin_memcpy(&w.b1[jb], par + kOffB1 + u, sizeof(f32x4));
+    __builtin_memcpy(&w.b2[jb], par + kOffB2 + u, sizeof(f32x4));
+    const bf16x4 w3 = load_bf4(wbf + kBfW3 + u);
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int u = jb * 16 + 4 * g + r;
-      w.b1[jb][r] = par[kOffB1 + u];
-      w.b2[jb][r] = par[kOffB2 + u];
-      w.w3[jb][r] = bf2f(wbf[kBfW3 + u]);
-    }
+    for (int r = 0; r < 4; r++) w.w3[jb][r] = bf2f((unsigned short)w3[r]);
   }
   w.b3 = par[kOffB3];
 #pragma unroll
