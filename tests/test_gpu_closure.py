@@ -72,6 +72,31 @@ def test_forward_tile_edges(lib, ctx, n):
         net.free()
 
 
+@pytest.mark.parametrize("n", [16, 70000])
+@pytest.mark.parametrize("z", [-87.5, -88.0, -88.5])
+def test_forward_keeps_small_activations(lib, ctx, n, z):
+    """silu(z) = z / (1 + e^-z) where 1 / (1 + e^-z) is subnormal and the quotient is
+    not: W2 = 0 gives every unit of the second layer z = b2, one of them is
+    scaled up by w3 = 2^120 to a term of at most 1.2. Bound: __expf rounds the
+    factor log2(e) and the product below 128, by up to 2^-18 each (5.3e-6 of
+    e^-z); the rest, of values below 2, stays below 3e-6."""
+    from oracle import mlp
+    feats = _features(max(n, 64))[:n]
+    net, p, mean, scale = _net(lib, ctx, _features(4096), out_scale=1.0)
+    net.free()
+    p[mlp.OFF_W2:mlp.OFF_B2] = 0
+    p[mlp.OFF_B2:mlp.OFF_W3] = z
+    p[mlp.OFF_W3:mlp.OFF_B3] = 0
+    p[mlp.OFF_W3 + 21] = 2.0 ** 120
+    p[mlp.OFF_B3] = 1
+    net = closure.Mlp(lib, ctx, p, mean, scale, 1.0)
+    try:
+        o = mlp.silu(np.float64(z)) * 2.0 ** 120 + 1
+        assert np.abs(net.forward(feats) - mlp.softplus(o)).max() <= 1e-5
+    finally:
+        net.free()
+
+
 @pytest.mark.parametrize("n,scratch_blocks", [(1003, 1024), (5000, 7)])
 def test_gradient_matches_oracle(lib, ctx, n, scratch_blocks):
     """scratch_blocks < tiles makes each block loop over several tiles."""
