@@ -250,6 +250,11 @@ __device__ inline float forward_tile_t(const FwdWeights& w, FeatFn feat, float& 
   return across_groups_sum(o) + w.b3;
 }
 
+// Turns of 16 kt samples that n samples take.
+__host__ __device__ inline unsigned fwd_turns(unsigned n, unsigned kt) {
+  return n / (16 * kt) + (n % (16 * kt) != 0);
+}
+
 // Runs the network over samples [0, n), 16 kT samples per wave and turn, and
 // calls done(sample, o) once per sample. kT = 4: lane group g finishes tile g
 // (whole waves store); kT = 1 spreads small batches over more waves.
@@ -260,7 +265,7 @@ __device__ inline void forward_all(unsigned n, const unsigned short* __restrict_
   const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
   FwdWeights w;
   load_weights(wbf, par, nm, w);
-  const unsigned nturns = (n + 16 * kT - 1) / (16 * kT);
+  const unsigned nturns = fwd_turns(n, kT);
   for (unsigned t = blockIdx.x; t < nturns; t += gridDim.x) {
     const unsigned base = t * 16 * kT;
     float o = 0.f;
@@ -276,9 +281,14 @@ __device__ inline void forward_all(unsigned n, const unsigned short* __restrict_
   }
 }
 
-// Resident waves of the inference kernels (4 per SIMD of 256 CUs); up to so many
-// tiles each wave takes one tile.
+// Resident waves of the inference kernels (4 per SIMD of 256 CUs); no more are
+// launched, and none without a turn.
 constexpr unsigned kFwdWaves = 4096;
+// Up to so many tiles each takes a wave of its own, above that a wave takes four and
+// loads the weights (10 KB) once for them. us of 16384 / 32768 / 40960 /
+// 65536 / 131072 samples: kT = 1 5.4 / 8.2 / 10.0 / 13.2 / 16.8, kT = 4 7.8 / 8.4 /
+// 8.9 / 9.6 / 13.1; k_sps_tau_learned, 32768 / 40960: 8.8 / 10.8 and 9.0 / 9.5.
+constexpr unsigned kFwdTiles1 = 2048;
 
 // nu[i] = out_scale * softplus(MLP(features[i])) for i in [0,n); features are
 // [n][11] FP32 rows.
@@ -640,11 +650,11 @@ int dsph_mlp_forward(dsph_ctx* ctx, const dsph_mlp* m, uint32_t n, const float* 
   if (!n) return DSPH_OK;
   DSPH_REQUIRE(ctx, m->d_params && m->d_wbf16 && d_features && d_out,
                "dsph_mlp_forward: null argument");
-  const unsigned ntiles = (n + 15) / 16;
   KTimer kt(ctx, "k_mlp_forward");
-  const auto kernel = ntiles <= kFwdWaves ? k_mlp_forward<1> : k_mlp_forward<4>;
-  kernel<<<std::min(ntiles, kFwdWaves), 64, 0, ctx->stream>>>(n, d_features, m->d_wbf16,
-                                                              m->d_params, make_norm(m), d_out);
+  const bool one = fwd_turns(n, 1) <= kFwdTiles1;
+  const auto kernel = one ? k_mlp_forward<1> : k_mlp_forward<4>;
+  kernel<<<std::min(fwd_turns(n, one ? 1 : 4), kFwdWaves), 64, 0, ctx->stream>>>(
+      n, d_features, m->d_wbf16, m->d_params, make_norm(m), d_out);
   DSPH_LAUNCHED(ctx, "k_mlp_forward");
   return DSPH_OK;
 }
@@ -693,10 +703,11 @@ int dsph_sps_tau_learned(dsph_ctx* ctx, const dsph_mlp* m, uint32_t np, uint32_t
   if (np <= npb) return DSPH_OK;
   DSPH_REQUIRE(ctx, m->d_params && m->d_wbf16 && d_velrho && d_velgrad && d_sps2strain && d_tau,
                "dsph_sps_tau_learned: null argument");
-  const unsigned n = np - npb, ntiles = (n + 15) / 16;
+  const unsigned n = np - npb;
   KTimer kt(ctx, "k_sps_tau_learned");
-  const auto kernel = ntiles <= kFwdWaves ? k_sps_tau_learned<1> : k_sps_tau_learned<4>;
-  kernel<<<std::min(ntiles, kFwdWaves), 64, 0, ctx->stream>>>(
+  const bool one = fwd_turns(n, 1) <= kFwdTiles1;
+  const auto kernel = one ? k_sps_tau_learned<1> : k_sps_tau_learned<4>;
+  kernel<<<std::min(fwd_turns(n, one ? 1 : 4), kFwdWaves), 64, 0, ctx->stream>>>(
       n, npb, blin, dp, (const float4*)d_velrho, d_velgrad, d_sps2strain, m->d_wbf16,
       m->d_params, make_norm(m), d_tau, d_nu);
   DSPH_LAUNCHED(ctx, "k_sps_tau_learned");

@@ -56,10 +56,11 @@ def test_forward_matches_oracle(lib, ctx, n):
         net.free()
 
 
-@pytest.mark.parametrize("n", [15, 17, 65535, 65537, 65600])
+@pytest.mark.parametrize("n", [15, 17, 32767, 32769, 32785, 65535, 65537, 65600, 262145])
 def test_forward_tile_edges(lib, ctx, n):
-    """Around one tile and around the change from one tile per wave and turn to
-    four (4096 tiles), bounds of test_forward_matches_oracle."""
+    """Around one tile, around the change from one tile per wave and turn to
+    four (2048 tiles), around 1024 turns of four and one more turn than there are
+    waves (4096), bounds of test_forward_matches_oracle."""
     from oracle import mlp
     feats = _features(max(n, 64), seed=n)[:n]
     net, p, mean, scale = _net(lib, ctx, _features(4096))
