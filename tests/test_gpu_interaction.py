@@ -181,6 +181,82 @@ def test_fluid_kernel_forms_equal_bitwise(make):
         np.testing.assert_array_equal(a, b)
 
 
+def _staged_and_rows(lib, ctx, c, tvisco, tddt, mdbc2=False, floating=False, poscell=None):
+    """(outputs of the kernels chosen by size and options, of the rows kernels,
+    boundary particles, sorted codes) for one interaction of case c: random tau,
+    with ``mdbc2`` random boundary modes and tangential velocities, with
+    ``floating`` two bodies, one lighter and one heavier than 1.2 fluid
+    particles. ``poscell``: changes a copy of the PosCell array in place."""
+    o, d, dcell, ps, cte, celldiv, be = _prepared(c)
+    st = o.stats()
+    n, npb, npbok = st["np"], st["npb"], st["npbok"]
+    rng = np.random.default_rng(2)
+    code, ps = d["code"].copy(), ps.copy()
+    if poscell:
+        poscell(ps, npb)
+    f32 = np.float32
+    dev = {"dcell": dcell, "poscell": ps, "velrho": d["velrho"],
+           "spstaurho2": (rng.standard_normal((n, 6)) * 1e-3).astype(f32)}
+    if mdbc2:
+        dev["boundmode"] = rng.integers(0, 3, n).astype(np.uint8)
+        dev["tangenvel"] = (rng.standard_normal((n, 3)) * 0.3).astype(f32)
+    if floating:
+        ft = (code & 0x1800) == 0x1000
+        assert ft.any()
+        code[ft] = (code[ft] & 0xf800) | rng.integers(0, 2, ft.sum()).astype(code.dtype)
+        dev["ftomassp"] = np.array([1.1 * c.massfluid, 1.3 * c.massfluid], f32)
+    dev["code"] = code
+    dev = {k: Dev(lib, ctx, a) for k, a in dev.items()}
+    bc = Dev(lib, ctx, be)
+    acte = to_cte(cte, tboundary=N.BC_MDBC if mdbc2 else N.BC_DBC)
+    assert lib.dsph_set_constants(ctx, C.byref(acte)) == 0
+    outs = []
+    for kernel in (N.FORCES_TILE, N.FORCES_ROWS):
+        out = {k: Dev.zeros(lib, ctx, s, f32) for k, s in (
+            ("ace", (n, 3)), ("ar", n), ("viscdt", n), ("sps2strain", (n, 6)))}
+        t = N.DsphInterParms()
+        t.tkernel, t.tvisco, t.tdensity = N.KERNEL_WENDLAND, tvisco, tddt
+        t.viscob, t.viscof = 0.01, 0.02
+        t.np, t.npb, t.npbok = n, npb, npbok
+        t.divdata = divdata(celldiv, bc, cte)
+        for k, a in (*dev.items(), *out.items()):
+            setattr(t, "d_" + k, a.ptr)
+        assert lib.dsph_ctx_set_option(ctx, N.OPT_FORCES_KERNEL, kernel) == 0
+        rc = lib.dsph_interaction_forces(ctx, C.byref(t))
+        assert lib.dsph_ctx_set_option(ctx, N.OPT_FORCES_KERNEL, N.FORCES_TILE) == 0
+        assert rc == 0, lib.dsph_last_error(ctx)
+        outs.append({k: a.get() for k, a in out.items()})
+    return (*outs, npb, code)
+
+
+def _strange_positions(ps, npb):
+    """Positions that are not finite, huge, or (finite) far outside the map in
+    about one of 50 particles, among them first ones of a wave."""
+    rng = np.random.default_rng(6)
+    for i0, i1 in ((0, npb), (npb, len(ps))):
+        pick = np.concatenate([rng.integers(i0, i1, (i1 - i0) // 50),
+                               i0 + 64 * rng.integers(0, (i1 - i0) // 64, (i1 - i0) // 500 + 5)])
+        for kind, i in enumerate(np.array_split(pick, 5)):
+            if kind < 4:
+                ps[i, rng.integers(0, 3, len(i))] = (np.inf, -np.inf, np.nan, 1e20)[kind]
+            else:
+                ps[i, 3] = (ps[i, 3].view(np.uint32) + np.uint32(300 << 19)).view(np.float32)
+
+
+@pytest.mark.parametrize("make", [lambda: casemod.dam_break(dp=0.02),
+                                  lambda: casemod.dam_break_2d(dp=0.0008)], ids=["team", "tile"])
+def test_strange_positions_leave_the_other_particles_alone(lib, ctx, make):
+    """A position that is not finite or far from its cell has no neighbours but
+    itself may be first of a wave: the sums of all particles are those
+    of the kernels in which each particle walks its own cells."""
+    a, b, npb, _ = _staged_and_rows(lib, ctx, perturbed_case(make()), N.VISCO_ARTIFICIAL,
+                                    N.DDT_DDT2FULL, poscell=_strange_positions)
+    assert np.isfinite(b["ace"]).all()
+    assert np.count_nonzero(b["ace"][npb:].any(1)) > 0.9 * (len(b["ace"]) - npb)
+    for k in a:
+        np.testing.assert_array_equal(a[k].view(np.uint32), b[k].view(np.uint32), err_msg=k)
+
+
 def test_tile_kernel_equals_rows_kernel_bitwise(lib, ctx):
     """Both fluid kernels sum the same pairs in the same order: identical bits."""
     c = perturbed_case(casemod.dam_break(dp=0.01), seed=3)
