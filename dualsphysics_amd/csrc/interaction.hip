@@ -140,9 +140,10 @@ struct GhostSums {
   float submerged;              // mDBC2: -sum V dr.gradW
 };
 static_assert(sizeof(GhostSums) == 24 * sizeof(float), "written lane by lane");
+static_assert(kGhostRec % 4 == 0, "records are whole float4");
 
 struct GhostLds {
-  float rec[kGhostBs * kGhostRec];
+  alignas(16) float rec[kGhostBs * kGhostRec];   // written float4 by float4
   GhostSums sums[kGhosts];
 };
 
