@@ -92,7 +92,7 @@ CASES = [
 ]
 
 
-@pytest.mark.parametrize("kernel", [N.FORCES_TILE, N.FORCES_ROWS], ids=["tile", "rows"])
+@pytest.mark.parametrize("kernel", [N.FORCES_TILE, N.FORCES_ROWS], ids=["staged", "rows"])
 @pytest.mark.parametrize("name,pert,tvisco,tddt,visco,viscob", CASES, ids=[x[0] for x in CASES])
 def test_interaction_parity(lib, ctx, name, pert, tvisco, tddt, visco, viscob, kernel):
     c = casemod.dam_break(dp=0.02)
@@ -130,7 +130,8 @@ def test_interaction_parity(lib, ctx, name, pert, tvisco, tddt, visco, viscob, k
 
 def _shuffled(c, m=None, seed=5):
     """The first m fluid particles (all by default) moved by up to 0.15 dp,
-    with random velocities, in random order."""
+    with random velocities, in random order; floating particles with random
+    velocities."""
     import dataclasses
     c = perturbed_case(c, seed=seed)
     rng = np.random.default_rng(seed)
@@ -140,6 +141,7 @@ def _shuffled(c, m=None, seed=5):
     if c.data2d:
         d[:, 1] = 0
     pos[nb:] = (pos[nb:] + d)[rng.permutation(m)]
+    c.velrho[nb - c.nfloat:nb, :3] = 0.3 * rng.standard_normal((c.nfloat, 3))
     return dataclasses.replace(c, idp=c.idp[:nb + m], pos=pos, velrho=c.velrho[:nb + m], nfluid=m)
 
 
@@ -155,9 +157,25 @@ FORMS = [("n%d" % m, lambda m=m: _shuffled(casemod.dam_break(dp=0.03), m))
     ("mdbc2", lambda: _shuffled(casemod.dam_break(dp=0.02, params=_P(
         tboundary=N.BC_MDBC, slipmode=N.SLIP_NOSLIP, tvisco=N.VISCO_LAMINAR, visco=1e-4)))),
     ("floating", lambda: casemod.dam_break_floating(dp=0.03)),
-    # Above the team kernel's sizes: the tile kernel.
+    ("sparse", lambda: _sparse(casemod.dam_break_2d(dp=0.0025), 400)),
+    # Above the team kernel's sizes (180k, 140k, 100k fluid particles in 3-D with
+    # artificial, laminar, SPS viscosity; three quarters in 2-D): the tile kernel.
     ("tile_2d", lambda: _shuffled(casemod.dam_break_2d(dp=0.0008))),
-]
+    ("tile_half_cells", lambda: _shuffled(casemod.dam_break(
+        dp=0.0072, params=_P(tvisco=N.VISCO_LAMINAR, visco=1e-4, cellmode=2)))),
+] + [("tile_n%d" % (m % 64), lambda m=m: _shuffled(casemod.dam_break_2d(dp=0.0008), m))
+     for m in (135040, 135041, 135055, 135057, 135103)]
+
+
+def _sparse(c, m):
+    """m fluid particles spread over the column (about one in four cells), so
+    the particles of a wave span many cells of a row."""
+    import dataclasses
+    nb = c.nbound
+    pick = nb + np.sort(np.random.default_rng(4).choice(c.nfluid, m, replace=False))
+    return _shuffled(dataclasses.replace(
+        c, idp=c.idp[:nb + m], pos=np.concatenate([c.pos[:nb], c.pos[pick]]),
+        velrho=np.concatenate([c.velrho[:nb], c.velrho[pick]]), nfluid=m))
 
 
 @pytest.mark.parametrize("make", [f for _, f in FORMS], ids=[n for n, _ in FORMS])
@@ -257,9 +275,48 @@ def test_strange_positions_leave_the_other_particles_alone(lib, ctx, make):
         np.testing.assert_array_equal(a[k].view(np.uint32), b[k].view(np.uint32), err_msg=k)
 
 
-def test_tile_kernel_equals_rows_kernel_bitwise(lib, ctx):
-    """Both fluid kernels sum the same pairs in the same order: identical bits."""
-    c = perturbed_case(casemod.dam_break(dp=0.01), seed=3)
+_ART, _LAM, _SPS = N.VISCO_ARTIFICIAL, N.VISCO_LAMINAR, N.VISCO_LAMINARSPS
+_FLOAT = lambda: _shuffled(casemod.dam_break_floating(dp=0.02))  # noqa: E731  teams
+_SMALL = lambda: _shuffled(casemod.dam_break(dp=0.02))  # noqa: E731  teams
+_LARGE = lambda: _shuffled(casemod.dam_break(dp=0.0072))   # noqa: E731  215k fluid particles: tile
+OPTIONS = [
+    ("floating_ddt1", _FLOAT, _ART, N.DDT_DDT, {"floating": True}),
+    ("floating_laminar_ddt2", _FLOAT, _LAM, N.DDT_DDT2, {"floating": True}),
+    ("floating_sps_ddt2full", _FLOAT, _SPS, N.DDT_DDT2FULL, {"floating": True}),
+    ("floating_sps_ddt1", _FLOAT, _SPS, N.DDT_DDT, {"floating": True}),
+    ("team_mdbc2_ddt1", _SMALL, _ART, N.DDT_DDT, {"mdbc2": True}),
+    ("team_mdbc2_laminar_ddt2", _SMALL, _LAM, N.DDT_DDT2, {"mdbc2": True}),
+    ("team_mdbc2_sps_ddt2full", _SMALL, _SPS, N.DDT_DDT2FULL, {"mdbc2": True}),
+    ("team_noddt", _SMALL, _ART, N.DDT_NONE, {}),
+    ("tile_ddt1", _LARGE, _ART, N.DDT_DDT, {}),
+    ("tile_ddt2", _LARGE, _ART, N.DDT_DDT2, {}),
+    ("tile_noddt", _LARGE, _LAM, N.DDT_NONE, {}),
+    ("tile_sps", _LARGE, _SPS, N.DDT_DDT2FULL, {}),
+    ("tile_mdbc2_ddt1", _LARGE, _ART, N.DDT_DDT, {"mdbc2": True}),
+    ("tile_mdbc2_laminar", _LARGE, _LAM, N.DDT_DDT2FULL, {"mdbc2": True}),
+    ("tile_mdbc2_sps_ddt2", _LARGE, _SPS, N.DDT_DDT2, {"mdbc2": True}),
+]
+
+
+@pytest.mark.parametrize("make,tvisco,tddt,options", [x[1:] for x in OPTIONS],
+                         ids=[x[0] for x in OPTIONS])
+def test_options_equal_bitwise(lib, ctx, make, tvisco, tddt, options):
+    """The rules of floating bodies (one lighter, one heavier than 1.2 fluid
+    particles), of mDBC2 boundaries and of the density diffusion terms in the team and tile
+    kernels: bits of the rows kernel, strain included."""
+    a, b, npb, code = _staged_and_rows(lib, ctx, make(), tvisco, tddt, **options)
+    assert np.abs(b["ace"][npb:]).max() > 0 and np.abs(b["ar"][npb:]).max() > 0
+    if tvisco == _SPS:
+        assert np.abs(b["sps2strain"][npb:]).max() > 0
+    for k in a:
+        np.testing.assert_array_equal(a[k].view(np.uint32), b[k].view(np.uint32), err_msg=k)
+
+
+@pytest.mark.parametrize("dp", [0.01, 0.0072], ids=["team", "tile"])
+def test_tile_kernel_equals_rows_kernel_bitwise(lib, ctx, dp):
+    """The staged kernels (80k fluid particles: teams, 215k: tile) and the rows
+    kernel sum the same pairs in the same order: identical bits."""
+    c = perturbed_case(casemod.dam_break(dp=dp), seed=3)
     gq, _, npb = _run_both(c, 1, 3, 0.01, 0.01, lib, ctx, kernel=N.FORCES_TILE)
     gr, _, _ = _run_both(c, 1, 3, 0.01, 0.01, lib, ctx, kernel=N.FORCES_ROWS)
     lib.dsph_ctx_set_option(ctx, N.OPT_FORCES_KERNEL, N.FORCES_TILE)
@@ -300,9 +357,9 @@ def test_sps_tau(lib, ctx):
 
 
 def test_boundary_kernel_forms_equal_bitwise(lib, ctx):
-    """The boundary interaction's tile form and its one-lane-per-particle
-    form give the same bits, and so does the automatic choice between them
-    over the interactions in which it times both (DSPH_OPT_BOUND_KERNEL)."""
+    """The boundary interaction with staged neighbours (form 1, and 0, the
+    default) and its one-lane-per-particle form (2) give the same bits
+    (DSPH_OPT_BOUND_KERNEL)."""
     c = perturbed_case(casemod.dam_break(dp=0.01), seed=4)
     o, d, dcell, poscell, cte, celldiv, be = _prepared(c)
     st = o.stats()
@@ -314,7 +371,7 @@ def test_boundary_kernel_forms_equal_bitwise(lib, ctx):
                                           ("velrho", d["velrho"]), ("code", d["code"]))}
     outs = []
     try:
-        for form, reps in ((N.BOUND_TILE, 1), (N.BOUND_ROWS, 1), (N.BOUND_AUTO, 7)):
+        for form, reps in ((N.BOUND_TILE, 1), (N.BOUND_ROWS, 1), (N.BOUND_AUTO, 1)):
             assert lib.dsph_ctx_set_option(ctx, N.OPT_BOUND_KERNEL, form) == 0
             for _ in range(reps):
                 ace = Dev.zeros(lib, ctx, (n, 3), np.float32)

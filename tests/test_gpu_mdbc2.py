@@ -86,7 +86,7 @@ def test_mdbc2_correction_matches_oracle(lib, ctx, name):
     np.testing.assert_array_equal(g_vr[:npb, :3], s["d"]["velrho"][:npb, :3])
 
 
-@pytest.mark.parametrize("kernel", [N.FORCES_TILE, N.FORCES_ROWS], ids=["tile", "rows"])
+@pytest.mark.parametrize("kernel", [N.FORCES_TILE, N.FORCES_ROWS], ids=["staged", "rows"])
 @pytest.mark.parametrize("tvisco,tddt", [(N.VISCO_LAMINAR, N.DDT_DDT2FULL),
                                          (N.VISCO_ARTIFICIAL, N.DDT_DDT2FULL),
                                          (N.VISCO_LAMINARSPS, N.DDT_DDT2)])

@@ -183,7 +183,8 @@ def test_tiny_and_empty_fluid(nfluid):
 def test_half_cells_match_oracle_and_kernels_agree():
     """CELLMODE_Half (cells of size h, 5x5 rows of 5 cells): GPU forces on a
     stepped state equal the FP32 oracle within 1e-5 (norm-wise), the neighbour
-    order is identical, and the tile and rows fluid kernels give the same bits."""
+    order is identical, and the staged (at this size: teams) and rows fluid kernels
+    give the same bits."""
     from dualsphysics_amd import _native as N
     from dualsphysics_amd.sim import SphGpuSingle
     from oracle.oracle import OracleSim
