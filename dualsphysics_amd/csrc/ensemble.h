@@ -101,7 +101,7 @@ int ens_forces_fluid(dsph_ctx* ctx, int variant, int tvisco, int tddt, bool eos7
                      float* viscdt, float* ar, float* ace);
 // Boundary interaction with neighbours staged in LDS (teams of four lanes per
 // particle; bmap64 has one entry per 64 boundary particles).
-int ens_forces_bound_tile(dsph_ctx* ctx, const EnsCase* cases, const EnsState* st,
+int ens_forces_bound_team(dsph_ctx* ctx, const EnsCase* cases, const EnsState* st,
                           const EnsBlock* bmap64, unsigned nblocks, const unsigned* dcell,
                           const float4* poscell, const float4* velrho, float* viscdt, float* ar);
 // bmap: one entry per block of bs boundary particles (bs = 64, 128, 192 or 256).

@@ -22,6 +22,11 @@
 //    order is unchanged.
 //  - k_forces_fluid_team: four lanes per particle, four consecutive pairs at a
 //    time, whose terms are then added in order (small and middle sizes).
+// One condition on "the same": the rows kernel takes the pairs within 2h among the
+// cells next to each particle's own, the other two those among the cells of a group
+// of particles. They differ by pairs two cells apart (2h or more, but for
+// rounding) whose FP32 distance rounds to 2h or less: the kernel gradient is nil
+// there, but their dot/r^2 enters the maximum viscdt.
 #include <cfloat>
 #include <cstring>
 #include <map>
@@ -515,10 +520,12 @@ __device__ __forceinline__ unsigned long long scan_tile(const float4* tile, unsi
 // and bit order, i.e. in the reference's summation order: the results equal
 // k_forces_fluid_rows bit for bit. Loads of the next pair are issued before
 // the arithmetic of the current one.
-// Bound by the VALU (1180 instructions per particle before the box test, a tenth of
-// them scanning) and the gathers. The box test halves the tiles to scan and lets a
-// ring of 8 tiles even out the lanes better than 12 tiles of whole rows did:
-// 6.1M particles 8.04 -> 7.12 ms (rings of 6 / 10 / 12: 7.38 / 7.30 / 7.32),
+// Bound by the VALU and the gathers, both near their limits at 6.1M particles: one
+// VALU instruction per 3.2 cycles and SIMD (1030 a particle; an FMA of vector
+// registers alone measured 2.9), and the texture data path of a CU busy 87 % of the
+// cycles (two 16-byte gathers a pair, 55 % of them from L1). The box test halves the
+// tiles to scan and lets a ring of 8 tiles even out the lanes better than 12 tiles of
+// whole rows did: 6.1M particles 8.04 -> 7.12 ms (rings of 6 / 10 / 12: 7.38 / 7.30 / 7.32),
 // 1.6M 2.15 -> 1.88 ms, a step of 3.0M particles in 2-D 1.99 -> 1.85 ms.
 // LDS of one wave of the tile kernel.
 template <unsigned kRing>
@@ -578,7 +585,6 @@ __device__ __forceinline__ void fluid_tile_body(unsigned p, bool valid, unsigned
       }
     }
   };
-  // k wave-uniform iterations; each lane pops up to k of its queued pairs.
   // Pops the next queued pair and issues its loads (32-bit offsets from the
   // array bases).
   // EOS7 (gamma = 7): the neighbour's {press, 1/rho} are evaluated from its
@@ -876,11 +882,13 @@ struct TeamArrays {
 // Why: with one lane per particle (tile kernel) a wave is a serial chain
 // of some 300 gathers and pair bodies, and below about 1e5 particles few
 // waves share the chip; four lanes per particle make four times the waves
-// with a quarter of the chain, and data in LDS replaces the gathers. Bound by
-// latency and VALU in about equal parts (VALU issue 77 % with 2 waves per
-// SIMD, 3 now). Dam breaks, artificial viscosity, tile -> team: 26k particles
-// 467 -> 115 us, 141k 511 -> 251 us, 357k 645 -> 573 us; boundary interaction
-// 207 -> 36, 238 -> 44 us and at 6.1M 570 -> 240 us.
+// with a quarter of the chain, and data in LDS replaces the gathers. Bound by the
+// latency of that chain: 80k fluid particles issue one VALU instruction per 6.6
+// cycles and SIMD, 10k (638 waves for 1024 SIMDs) one per 27; texture data path 32
+// and 10 % of the cycles, LDS bank conflicts 7 and 2 %. us, tile -> team (dam breaks,
+// artificial viscosity): 26k particles, 10k of them fluid, 321 -> 111; 141k (80k)
+// 381 -> 253; 253k (157k) 428 -> 414; 357k (234k) 531 -> 578. Boundary interaction,
+// one lane per particle -> team: 26k 229 -> 46, 141k 243 -> 49, 6.1M 406 -> 196.
 // Computed share of busy lanes in the pair body for particles in lattice order:
 // ring of 128 77 %, 192 86 %, 256 94 % (but a wave less per SIMD).
 constexpr unsigned kTeam = 4;             // lanes per particle
@@ -1201,7 +1209,7 @@ __device__ __forceinline__ void team_body(unsigned pw, unsigned n, unsigned pini
   };
 
   struct Nb { float4 ps, vr; float pr; P2x x; bool has; };
-  // its rounds of four consecutive hits per team.
+  // Evaluates the next four hits of every team, one a lane, its times.
   auto process = [&](auto kb, const PairK& pk, int its) {
     constexpr bool KB = decltype(kb)::value;
     auto fetch = [&](Nb& b) {
@@ -1969,7 +1977,7 @@ int ens_forces_bound(dsph_ctx* ctx, const EnsCase* cases, const EnsState* st,
   return DSPH_OK;
 }
 
-int ens_forces_bound_tile(dsph_ctx* ctx, const EnsCase* cases, const EnsState* st,
+int ens_forces_bound_team(dsph_ctx* ctx, const EnsCase* cases, const EnsState* st,
                           const EnsBlock* bmap64, unsigned nblocks, const unsigned* dcell,
                           const float4* poscell, const float4* velrho, float* viscdt, float* ar) {
   if (!nblocks) return DSPH_OK;
@@ -1993,12 +2001,12 @@ int dsph_ctx_set_option(dsph_ctx* ctx, int key, int value) {
   if (!ctx) return DSPH_E_ARG;
   switch (key) {
     case DSPH_OPT_FORCES_KERNEL:
-      DSPH_REQUIRE(ctx, value == 0 || value == 1, "forces kernel must be 0 (tile) or 1 (rows)");
+      DSPH_REQUIRE(ctx, value == 0 || value == 1, "forces kernel must be 0 (staged) or 1 (rows)");
       ctx->forces_kernel = value;
       return DSPH_OK;
     case DSPH_OPT_BOUND_KERNEL:
       DSPH_REQUIRE(ctx, value >= 0 && value <= 2,
-                   "boundary kernel must be 0 (auto), 1 (tile) or 2 (rows)");
+                   "boundary kernel must be 0 (auto), 1 (staged) or 2 (rows)");
       ctx->bound_kernel = value;
       return DSPH_OK;
     default: return set_error(ctx, DSPH_E_ARG, "unknown option");
@@ -2070,8 +2078,9 @@ int interaction_forces(dsph_ctx* ctx, const dsph_inter_parms* t, float2* press) 
   if (t->npbok) {
     KTimer kt(ctx, "k_forces_bound");
     if (ctx->forces_kernel == 0 && ctx->bound_kernel != 2) {
-      // Teams beat one lane per particle at every size (us, dam break dp
-      // 0.02 / 0.01 / 0.0025: 36 / 44 / 240 against 207 / 238 / 350).
+      // Teams beat one lane per particle at every size (us, dam breaks of 26k / 141k /
+      // 6.1M particles 46 / 49 / 196 against 229 / 243 / 406, wave flume of 1.1M
+      // 128 against 326).
       const unsigned g = grid_for(t->npbok, kTeamP);
       const TeamArrays A = team_arrays(t, press);
       if (t->d_ftomassp)

@@ -21,8 +21,8 @@
 // kernel) on a one-workgroup-per-wave grid, then the best tile variant in its
 // persistent form over chunks of 1, 2 or 4 waves of particles per counter
 // fetch and grids of 10, 20 or 40 waves per CU; and the boundary kernel:
-// one lane per particle in blocks of 64, 128 or 256, or the tile form (one
-// wave per 64 boundary particles). All shapes give identical results.
+// one lane per particle in blocks of 64, 128 or 256, or the form with staged
+// neighbours (teams of four lanes per particle). All shapes give identical results.
 #include <hip/hip_runtime.h>
 #include <memory>
 #include "ensemble.h"
@@ -61,7 +61,7 @@ struct dsph_ens {
   // Boundary block maps, one per candidate block size.
   EnsBlock* d_bmaps[kNumBoundBs] = {nullptr, nullptr, nullptr};
   unsigned nbblocks[kNumBoundBs] = {0, 0, 0};
-  unsigned ibs = 1;  // kBoundBs[ibs] = 128 until tuned; kNumBoundBs = the tile form
+  unsigned ibs = 1;  // kBoundBs[ibs] = 128 until tuned; kNumBoundBs = staged neighbours
   float bound_ms[kNumBoundBs + 1] = {0, 0, 0, 0};
   unsigned ncu = 256;
   unsigned* d_ctr = nullptr;  // kNumXcd counters per bucket (persistent fluid kernel)
@@ -363,7 +363,7 @@ struct dsph_ens {
   // of kBoundBs[s]; s == kNumBoundBs the form with staged neighbours over the 64-blocks.
   void bound(unsigned s) {
     if (s == kNumBoundBs)
-      chk(dsph::ens_forces_bound_tile(ctx, d_cases, d_st, d_bmaps[0], nbblocks[0], dcell,
+      chk(dsph::ens_forces_bound_team(ctx, d_cases, d_st, d_bmaps[0], nbblocks[0], dcell,
                                       (const float4*)poscell, (const float4*)velrho, viscdt, ar),
           "bound interaction");
     else

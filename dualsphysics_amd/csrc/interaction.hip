@@ -126,8 +126,10 @@ __device__ inline double mdbc_det_inv(bool sim2d, const M4d& a, M4d& inv) {
 // sum runs in the order of one lane walking the rows, with its roundings:
 // identical bits. One lane per ghost node was a serial chain of some 700
 // gathers on few waves. mDBC2 step of 200k particles 2.04 -> 1.50 ms (78k
-// boundary particles: 428 us a call before); where many walls fill the chip
-// (wave flume, 0.6M boundary particles) 567 -> 518 us, bound by the VALU.
+// boundary particles: 428 -> 145 us a call); where many walls fill the chip
+// (wave flume, 0.6M boundary particles) 567 -> 518 us: the texture data path is busy
+// 84 % of the cycles (96 % of its requests hit L1), LDS bank conflicts take 24 %, and
+// a SIMD issues one VALU instruction per 4.6 cycles.
 constexpr unsigned kGhostLanes = 16, kGhosts = 16;   // lanes per ghost, ghosts per workgroup
 constexpr unsigned kGhostBs = kGhostLanes * kGhosts;
 constexpr unsigned kGhostRec = 20;   // floats per record: F[4], D[4], Q[8], {-volume}
