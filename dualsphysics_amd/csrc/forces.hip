@@ -654,7 +654,8 @@ __device__ __forceinline__ void fluid_tile_body(unsigned p, bool valid, unsigned
     const float q1x = c.pcs * float(pfx - rfx) + q.ps.x, q1y = c.pcs * float(pfy - rfy) + q.ps.y,
                 q1z = c.pcs * float(pfz - rfz) + q.ps.z;
     // A position that is not finite, or whose square may not be, stays out of the
-    // box: all neighbours of the group go to its exact test.
+    // box: all neighbours of the group pass (0 + |q2|^2 <= inf; not a position that
+    // is not finite) and go to its exact test.
     const bool near = member && q1x * q1x + q1y * q1y + q1z * q1z < 1e30f, far = member && !near;
     const float bx0 = wave_min_f32(near ? q1x : FLT_MAX),
                 bx1 = -wave_min_f32(near ? -q1x : FLT_MAX);
@@ -669,8 +670,9 @@ __device__ __forceinline__ void fluid_tile_body(unsigned p, bool valid, unsigned
     const float qm = sqrtf(ex * ex + ey * ey + ez * ez) + 1.01f * sqrtf(c.ks2);
     const float reach2 = c.ks2 * 1.00004f + 2.0e-6f * qm * qm;
     const float box2 = __ballot(far) ? __builtin_inff() : reach2;
-    const float thr = reach2 - s1;
-    const float m2x = -2.f * qx, m2y = -2.f * qy, m2z = -2.f * qz;
+    const float thr = far ? __builtin_inff() : reach2 - s1;
+    const float m2x = far ? 0.f : -2.f * qx, m2y = far ? 0.f : -2.f * qy,
+                m2z = far ? 0.f : -2.f * qz;
     const int ny = Y1 - Y0, nrows = ny * (Z1 - Z0);
     // Rows of the group, fluid cells then boundary cells, one a lane (18 in
     // all, or 50 of half cells); 64 neighbours of a row at a time. Those near
@@ -736,9 +738,8 @@ __device__ __forceinline__ void fluid_tile_body(unsigned p, bool valid, unsigned
         const unsigned nt = min(fill, kTile);
         unsigned long long hm = 0;
         if (member)
-          hm = (scan_tile(lds.tile + (wt & 1) * kTile, (nt + kScanBlock - 1) / kScanBlock, m2x, m2y,
-                          m2z, thr) |
-                (far ? ~0ull : 0ull)) &
+          hm = scan_tile(lds.tile + (wt & 1) * kTile, (nt + kScanBlock - 1) / kScanBlock, m2x, m2y,
+                         m2z, thr) &
                (~0ull >> (kTile - nt));
         masks[wt % kRing][lane] = hm;
         if (len == 0) {
