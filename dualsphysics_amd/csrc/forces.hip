@@ -655,7 +655,9 @@ __device__ __forceinline__ void fluid_tile_body(unsigned p, bool valid, unsigned
                 q1z = c.pcs * float(pfz - rfz) + q.ps.z;
     // A position that is not finite, or whose square may not be, stays out of the
     // box: all neighbours of the group pass (0 + |q2|^2 <= inf; not a position that
-    // is not finite) and go to its exact test.
+    // is not finite) and go to its exact test. (A pass of steps at 6.1M particles,
+    // without any of this / so: 373.1 / 373.9 ms; all bits or-ed into the hits of each
+    // tile instead, in another run: 364.9 / 367.8.)
     const bool near = member && q1x * q1x + q1y * q1y + q1z * q1z < 1e30f, far = member && !near;
     const float bx0 = wave_min_f32(near ? q1x : FLT_MAX),
                 bx1 = -wave_min_f32(near ? -q1x : FLT_MAX);
